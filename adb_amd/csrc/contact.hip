@@ -32,95 +32,18 @@
 // the Jacobi tolerance (the reference's own test sees the nine rounding-level
 // eigenvalues of the translations).
 //
-// Kernel-level API (k_hess_api, the abdtk functions): one 16-lane group per
-// contact, four contacts per wavefront, lane j < 12 owning column j of the
-// 12 x 12 Hessian; its 9 x 9 projection is parallel cyclic Jacobi (5 disjoint
-// rotations per round, 9 rounds per sweep over 10 slots, slot 9 idle) on the
-// matrix staged in LDS.
+// Kernel-level API (the abdtk functions): k_hess_api, one thread per contact
+// in the five-coordinate frame of terms.h; mollified edge pairs in
+// k_hess_moll.  Against the 16-lane groups with a 9 x 9 Jacobi in LDS that
+// they replaced (a barrier per round of rotations): 1021 PT contacts 114 ->
+// 22 us a call, 2e5 EE contacts (a tenth mollified) 4458 -> 200 us.
 #include <cstdio>
 #include <algorithm>
 #include "dmath.h"
+#include "terms.h"
 #include "world.h"
 
 namespace adb {
-
-__constant__ signed char kRR9[9][5][2] = {
-    {{0, 9}, {1, 8}, {2, 7}, {3, 6}, {4, 5}}, {{0, 1}, {2, 9}, {3, 8}, {4, 7}, {5, 6}},
-    {{0, 2}, {1, 3}, {4, 9}, {5, 8}, {6, 7}}, {{0, 3}, {2, 4}, {1, 5}, {6, 9}, {7, 8}},
-    {{0, 4}, {3, 5}, {2, 6}, {1, 7}, {8, 9}}, {{0, 5}, {4, 6}, {3, 7}, {2, 8}, {1, 9}},
-    {{0, 6}, {5, 7}, {4, 8}, {3, 9}, {1, 2}}, {{0, 7}, {6, 8}, {5, 9}, {1, 4}, {2, 3}},
-    {{0, 8}, {7, 9}, {1, 6}, {2, 5}, {3, 4}}};
-
-// Helmert basis of the complement of (1, 1, 1, 1) / 2 in R^4
-#define HS2 0.70710678118654752440
-#define HS6 0.40824829046386301637
-#define HS12 0.28867513459481288225
-__constant__ double kHel[3][4] = {{HS2, -HS2, 0.0, 0.0}, {HS6, HS6, -2.0 * HS6, 0.0}, {HS12, HS12, HS12, -3.0 * HS12}};
-
-constexpr int GL = 16;        // lanes per contact
-constexpr int CPW = 4;        // contacts per 64-lane workgroup
-constexpr int LDH = 13;       // padded leading dimensions in LDS
-constexpr int LDK = 11;
-constexpr int MAX_SWEEPS = 15;
-// Jacobi stops when the squared off-diagonal Frobenius norm is below this
-// fraction of the total (off-diagonal entries ~1e-12 relative: rounding-level
-// for the projected Hessian, and reachable in a few sweeps, unlike 1e-30,
-// which sits at the FP64 noise floor of the rotations themselves)
-constexpr double JACOBI_TOL = 1e-24;
-// rotations of off-diagonal entries below JACOBI_SKIP * |A|_F are skipped: 36
-// such entries add at most 36e-28 |A|_F^2 to the off-diagonal sum, far below
-// the stop test, and late sweeps then cost little
-constexpr double JACOBI_SKIP = 1e-14;
-// Reciprocal and reciprocal square root from the hardware approximations,
-// each refined by two Newton steps (each step doubles the correct bits).
-// The Jacobi rotation parameters need no correct rounding, and this chain is
-// several times shorter than IEEE division and square root.
-__device__ __forceinline__ double rcp_r(double x) {
-    double y = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, y, 1.0); y = fma(y, e, y);
-    e = fma(-x, y, 1.0); return fma(y, e, y);
-}
-__device__ __forceinline__ double rsq_r(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-    const double h = 0.5 * x;
-    double e = fma(-h * y, y, 0.5); y = fma(y, e, y);
-    e = fma(-h * y, y, 0.5); return fma(y, e, y);
-}
-// The same with one Newton step: where only the rotation angle depends on
-// the value, an error there leaves a residual of that relative size in the
-// annihilated entry (removed by the next sweep), not a non-orthogonal rotation.
-__device__ __forceinline__ double rcp_r1(double x) {
-    const double y = __builtin_amdgcn_rcp(x);
-    return fma(y, fma(-x, y, 1.0), y);
-}
-__device__ __forceinline__ double rsq_r1(double x) {
-    const double y = __builtin_amdgcn_rsq(x);
-    return fma(y, fma(-(0.5 * x) * y, y, 0.5), y);
-}
-// Jacobi rotation annihilating a_pq (Golub and Van Loan, Algorithm 8.5.1):
-// tau = (a_qq - a_pp) / (2 a_pq), t = sign(tau) / (|tau| + sqrt(1 + tau^2)),
-// c = 1 / sqrt(1 + t^2), s = t c; after it a_pp' = a_pp - t a_pq, a_qq' = a_qq + t a_pq.
-// t sets only the angle (one Newton step each); c keeps two, so that
-// c^2 + s^2 = 1 to rounding and the accumulated rotations stay orthogonal.
-__device__ __forceinline__ void jacobi_cs(double app, double aqq, double apq, double& c, double& s, double& t) {
-    const double tau = (aqq - app) * (0.5 * rcp_r1(apq));
-    if (fabs(tau) > 1e150) {
-        t = 0.5 * rcp_r1(tau);
-    } else {
-        const double x = fma(tau, tau, 1.0);
-        t = (tau >= 0 ? 1.0 : -1.0) * rcp_r1(fma(x, rsq_r1(x), fabs(tau)));      // x rsq(x) = sqrt(x)
-    }
-    c = rsq_r(fma(t, t, 1.0));
-    s = t * c;
-}
-
-struct GroupLDS {
-    double H[12][LDH];
-    double A[9][LDK];
-    double V[9][LDK];
-    double cs[5][2];
-    double g[12];
-};
 
 struct KParams {
     double d_hat, kappa, eps_x;
@@ -128,152 +51,6 @@ struct KParams {
     double mu, eps_v, max_uk;
     int pt_fric, ee_fric;
 };
-
-__device__ __forceinline__ double sel12(const double a[12], int j) {
-    double r = 0.0;
-#pragma unroll
-    for (int k = 0; k < 12; k++) r = (k == j) ? a[k] : r;
-    return r;
-}
-__device__ __forceinline__ double sel4(double a0, double a1, double a2, double a3, int j) {
-    return j == 0 ? a0 : (j == 1 ? a1 : (j == 2 ? a2 : a3));
-}
-
-// ---------------------------------------------------------------- PSD (group)
-// Input: the symmetric vertex-space Hessian in S.H (all 64 lanes must call:
-// barriers).  HOUT = false: S.H is projected in place, and left unchanged when
-// the matrix is already PSD or `on` is false.  HOUT = true: S.A receives the
-// Helmert-coordinate matrix K = Q H Q^T, replaced by its projection
-// V diag(max(w, 0)) V^T when `on`.
-// KIN = true: S.A already holds K (S.H is not read).
-template <bool HOUT, bool KIN = false>
-__device__ __forceinline__ void group_psd(GroupLDS& S, int lane, bool on) {
-    // K = Q H Q^T: lane u = (b, j) < 9 builds column u
-    if (!KIN && lane < 9) {
-        const int b = lane / 3, j = lane % 3;
-        double hb[4];
-#pragma unroll
-        for (int l = 0; l < 4; l++) hb[l] = kHel[b][l];
-        double t[4][3];
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-#pragma unroll
-            for (int i = 0; i < 3; i++) {
-                double s = 0.0;
-#pragma unroll
-                for (int l = 0; l < 4; l++) s += hb[l] * S.H[3 * k + i][3 * l + j];
-                t[k][i] = s;
-            }
-#pragma unroll
-        for (int a = 0; a < 3; a++)
-#pragma unroll
-            for (int i = 0; i < 3; i++) {
-                double s = 0.0;
-#pragma unroll
-                for (int k = 0; k < 4; k++) s += kHel[a][k] * t[k][i];
-                S.A[3 * a + i][lane] = s;
-            }
-    }
-    if (lane < 9) {
-#pragma unroll
-        for (int r = 0; r < 9; r++) S.V[r][lane] = (r == lane) ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    for (int sweep = 0; sweep < MAX_SWEEPS; sweep++) {
-        double off = 0.0, tot = 0.0;
-        if (lane < 9) {
-#pragma unroll
-            for (int r = 0; r < 9; r++) { double a = S.A[r][lane]; tot += a * a; if (r != lane) off += a * a; }
-        }
-        for (int m = 8; m >= 1; m >>= 1) { off += __shfl_xor(off, m, GL); tot += __shfl_xor(tot, m, GL); }
-        const bool conv = !on || off <= JACOBI_TOL * tot || off == 0.0;
-        if (__all(conv)) break;
-        for (int rd = 0; rd < 9; rd++) {
-            if (lane < 5) {
-                const int p = kRR9[rd][lane][0], q = kRR9[rd][lane][1];
-                double c = 1.0, s = 0.0;
-                if (!conv && q < 9) {
-                    const double apq = S.A[p][q];
-                    if (apq != 0.0) {
-                        const double app = S.A[p][p], aqq = S.A[q][q];
-                        double t;
-                        jacobi_cs(app, aqq, apq, c, s, t);
-                    }
-                }
-                S.cs[lane][0] = c; S.cs[lane][1] = s;
-            }
-            __syncthreads();
-            if (!conv && lane < 9) {          // A <- A J and V <- V J: lane owns row `lane`
-#pragma unroll
-                for (int k = 0; k < 5; k++) {
-                    const int p = kRR9[rd][k][0], q = kRR9[rd][k][1];
-                    if (q < 9) {
-                        const double c = S.cs[k][0], s = S.cs[k][1];
-                        const double ap = S.A[lane][p], aq = S.A[lane][q];
-                        S.A[lane][p] = fma(c, ap, -s * aq); S.A[lane][q] = fma(s, ap, c * aq);
-                        const double vp = S.V[lane][p], vq = S.V[lane][q];
-                        S.V[lane][p] = fma(c, vp, -s * vq); S.V[lane][q] = fma(s, vp, c * vq);
-                    }
-                }
-            }
-            __syncthreads();
-            if (!conv && lane < 9) {          // A <- J^T A: lane owns column `lane`
-#pragma unroll
-                for (int k = 0; k < 5; k++) {
-                    const int p = kRR9[rd][k][0], q = kRR9[rd][k][1];
-                    if (q < 9) {
-                        const double c = S.cs[k][0], s = S.cs[k][1];
-                        const double ap = S.A[p][lane], aq = S.A[q][lane];
-                        S.A[p][lane] = fma(c, ap, -s * aq); S.A[q][lane] = fma(s, ap, c * aq);
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    }
-    double w[9];
-    double wmin = 0.0;
-#pragma unroll
-    for (int k = 0; k < 9; k++) { w[k] = S.A[k][k]; wmin = k == 0 ? w[k] : fmin(wmin, w[k]); }
-    const bool project = HOUT ? on : (on && wmin < 0.0);
-    __syncthreads();
-    // P(K) = V diag(max(w, 0)) V^T, column `lane`, into A
-    if (project && lane < 9) {
-#pragma unroll
-        for (int r = 0; r < 9; r++) {
-            double s = 0.0;
-#pragma unroll
-            for (int k = 0; k < 9; k++) s += S.V[r][k] * fmax(w[k], 0.0) * S.V[lane][k];
-            S.A[r][lane] = s;
-        }
-    }
-    __syncthreads();
-    if (HOUT) return;
-    // H_psd = Q^T P(K) Q: lane v = (l, j) < 12 builds column v
-    if (project && lane < 12) {
-        const int l = lane / 3, j = lane % 3;
-        double s_ai[3][3];
-#pragma unroll
-        for (int a = 0; a < 3; a++)
-#pragma unroll
-            for (int i = 0; i < 3; i++) {
-                double s = 0.0;
-#pragma unroll
-                for (int b = 0; b < 3; b++) s += kHel[b][l] * S.A[3 * a + i][3 * b + j];
-                s_ai[a][i] = s;
-            }
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-#pragma unroll
-            for (int i = 0; i < 3; i++) {
-                double s = 0.0;
-#pragma unroll
-                for (int a = 0; a < 3; a++) s += kHel[a][k] * s_ai[a][i];
-                S.H[3 * k + i][lane] = s;
-            }
-    }
-    __syncthreads();
-}
 
 // ---------------------------------------------------------------- barrier Hessian column
 // Contact geometry and barrier scalars, computed redundantly by every lane of
@@ -347,45 +124,6 @@ __device__ __forceinline__ double grad_m(const Geo& G, int k, int i) {
     const double sz = (k == 3 ? 1.0 : 0.0) - (k == 2 ? 1.0 : 0.0);
     return G.m1 * (sy * G.mc.grad(0, i) + sz * G.mc.grad(1, i));
 }
-// column j of the barrier Hessian (model/core_ipc.cpp:36-43,70-80) and g_j
-__device__ __forceinline__ void barrier_column(const Geo& G, int j, double (*H)[LDH], double& gj) {
-    const int l = j / 3, c = j % 3;
-    const double gdj = grad_d(G, l, c), gmj = grad_m(G, l, c);
-    const double syl = (l == 1 ? 1.0 : 0.0) - (l == 0 ? 1.0 : 0.0), szl = (l == 3 ? 1.0 : 0.0) - (l == 2 ? 1.0 : 0.0);
-    const double gxj = syl * G.mc.grad(0, c) + szl * G.mc.grad(1, c);
-#pragma unroll 1
-    for (int k = 0; k < 4; k++)
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-            // d^2 d / dx_(k,i) dx_(l,c) from the reduced Hessian
-            double hd = 0.0;
-#pragma unroll
-            for (int m = 0; m < 3; m++)
-#pragma unroll
-                for (int n = 0; n < 3; n++)
-                    if (m < G.map.nr && n < G.map.nr) {
-                        const double sg = red_sign(G.map, m, k) * red_sign(G.map, n, l);
-                        if (sg != 0.0) hd += sg * G.rd.hess(m, i, n, c);
-                    }
-            const double gdi = grad_d(G, k, i);
-            if (!G.is_ee) {
-                H[3 * k + i][j] = hd * G.B1 + gdi * gdj * G.B2;
-            } else {
-                double hm = 0.0, gmi = 0.0;
-                if (G.m2 != 0.0) {
-                    const double syk = (k == 1 ? 1.0 : 0.0) - (k == 0 ? 1.0 : 0.0), szk = (k == 3 ? 1.0 : 0.0) - (k == 2 ? 1.0 : 0.0);
-                    const double hx = syk * syl * G.mc.hess(0, i, 0, c) + syk * szl * G.mc.hess(0, i, 1, c)
-                                    + szk * syl * G.mc.hess(1, i, 0, c) + szk * szl * G.mc.hess(1, i, 1, c);
-                    const double gxi = syk * G.mc.grad(0, i) + szk * G.mc.grad(1, i);
-                    hm = G.m2 * gxi * gxj + G.m1 * hx;
-                    gmi = G.m1 * gxi;
-                }
-                H[3 * k + i][j] = hm * G.B0 + G.B1 * (gmi * gdj + gdi * gmj) + G.m * (G.B2 * gdi * gdj + G.B1 * hd);
-            }
-        }
-    gj = G.is_ee ? G.m * gdj * G.B1 + gmj * G.B0 : gdj * G.B1;
-}
-
 // vertex-space gradient entry j = (point, component) < 12 (model/core_ipc.cpp:36-43,70-80)
 __device__ __forceinline__ double barrier_grad(const Geo& G, int j) {
     const int l = j / 3, c = j % 3;
@@ -394,7 +132,6 @@ __device__ __forceinline__ double barrier_grad(const Geo& G, int j) {
 }
 
 // ---------------------------------------------------------------- friction setup
-__device__ __forceinline__ d3 unit(d3 a) { double l = sqrt(sqn(a)); return mk(a.x / l, a.y / l, a.z / l); }
 __device__ __forceinline__ void basis_pp(d3 p0, d3 p1, d3& c0, d3& c1) {
     d3 d = p1 - p0;
     d3 cx = cross(mk(1, 0, 0), d), cy = cross(mk(0, 1, 0), d);
@@ -487,35 +224,191 @@ __device__ __forceinline__ void friction_M(double u0, double u1, double lam, con
 }
 
 // ---------------------------------------------------------------- kernel-level API
-// H and g of IPC::ipc_hess_{pt,ee}_12x12 for n independent inputs.
+// H and g of IPC::ipc_hess_{pt,ee}_12x12 for n independent inputs, one thread
+// each: the Hessian in the contact's five-coordinate frame (terms.h),
+// projected there by a 5 x 5 Jacobi in registers, and expanded to the 12 x 12
+// blocks as it is stored (column by column, 16-byte stores: a lane's column
+// is 96 consecutive bytes).  Bound by the 1.3 KB stored per contact for large
+// n, by the Jacobi's dependent chain for small n (64-lane workgroups, so that
+// a few contacts spread over the CUs).  Mollified edge pairs are left to
+// k_hess_moll.
+__device__ __forceinline__ void load_points(const double* __restrict__ x, int e, d3& P0, d3& P1, d3& P2, d3& P3) {
+    const dd8* p = reinterpret_cast<const dd8*>(x + 12 * (size_t)e);
+    dd8 v[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) v[k] = p[k];
+    P0 = mk(v[0].x, v[0].y, v[1].x); P1 = mk(v[1].y, v[2].x, v[2].y);
+    P2 = mk(v[3].x, v[3].y, v[4].x); P3 = mk(v[4].y, v[5].x, v[5].y);
+}
 template <int IS_EE>
-__global__ __launch_bounds__(64) void k_hess_api(KParams kp, int n, const double* __restrict__ x,
-                                                   const int* __restrict__ type, const double* __restrict__ dist,
-                                                   double* __restrict__ H, double* __restrict__ g, double* __restrict__ moll) {
-    __shared__ GroupLDS lds[CPW];
-    const int grp = threadIdx.x / GL, lane = threadIdx.x % GL;
-    const int e = blockIdx.x * CPW + grp;
-    const bool valid = e < n;
-    GroupLDS& L = lds[grp];
-    Geo G;
-    double gj = 0.0;
-    double mval = 1.0;
-    if (valid) {
-        const double* xe = x + 12 * (size_t)e;
-        G.p0 = ld3(xe); G.p1 = ld3(xe + 3); G.p2 = ld3(xe + 6); G.p3 = ld3(xe + 9);
-        G.is_ee = IS_EE; G.type = type[e]; G.d = dist[e];
-        geo_init(G, kp);
-        mval = G.m;
-        if (lane < 12) barrier_column(G, lane, L.H, gj);
-    } else if (lane < 12) {
-        for (int i = 0; i < 12; i++) L.H[i][lane] = 0.0;
+__global__ __launch_bounds__(64) void k_hess_api(KParams kp, int n, const double* __restrict__ x, const int* __restrict__ type,
+                                                 const double* __restrict__ dist, double* __restrict__ H, double* __restrict__ g,
+                                                 double* __restrict__ moll) {
+    const int e = blockIdx.x * 64 + threadIdx.x;
+    if (e >= n) return;
+    d3 P0, P1, P2, P3;
+    load_points(x, e, P0, P1, P2, P3);
+    if (IS_EE) {
+        Mollifier q;
+        if (mollifier(kp.eps_x, P0, P1, P2, P3, q)) return;
+        if (moll) moll[e] = 1.0;
+    }
+    const double d = dist[e];
+    const double B1 = barrier_d1(d, kp.d_hat, kp.kappa), B2 = barrier_d2(d, kp.d_hat, kp.kappa);
+    Frame F;
+    contact_frame(IS_EE, type[e], P0, P1, P2, P3, F);
+    double M[15];
+    frame_matrix(F, B1, B2, M);
+    if (kp.psd) {
+        double V[25];
+        jacobi_packed<5>(M, V);
+        project_packed<5>(M, V);
+    }
+    const double gs = 2.0 * B1 * F.delta;
+    double* ge = g + 12 * (size_t)e;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) ge[3 * k + i] = gs * F.gam[k] * cmp(F.n, i);
+    // entry ((k, i), (l, j)) = gh_k gh_l T_ij + gh_k h_l,i n_j + n_i gh_l h_k,j + N_kl n_i n_j:
+    // T the tangential 3 x 3 matrix, h_l = sum_t M(t, y) (Q_l) f_t, N = Q M(y, y) Q^T
+    double gh[4], N[4][4], T[6];
+    d3 h[4];
+    const double ign = 1.0 / F.gn;
+    double c1[4], c2[4];
+    {
+        const double y1[3] = {M[PK_<5>(0, 2)], M[PK_<5>(0, 3)], M[PK_<5>(0, 4)]};
+        const double y2[3] = {M[PK_<5>(1, 2)], M[PK_<5>(1, 3)], M[PK_<5>(1, 4)]};
+        unhelmert(y1, F.in, c1);
+        unhelmert(y2, F.in, c2);
+        double R[3][4];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            const double ya[3] = {M[PK_<5>(2 + a, 2)], M[PK_<5>(2 + a, 3)], M[PK_<5>(2 + a, 4)]};
+            unhelmert(ya, F.in, R[a]);
+        }
+#pragma unroll
+        for (int l = 0; l < 4; l++) {
+            const double col[3] = {R[0][l], R[1][l], R[2][l]};
+            unhelmert(col, F.in, N[l]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        gh[k] = F.gam[k] * ign;
+        h[k] = c1[k] * F.f1 + c2[k] * F.f2;
+    }
+    {
+        const double a = M[PK_<5>(0, 0)], b = M[PK_<5>(0, 1)], c = M[PK_<5>(1, 1)];
+        int u = 0;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = i; j < 3; j++) {
+                const double f1i = cmp(F.f1, i), f1j = cmp(F.f1, j), f2i = cmp(F.f2, i), f2j = cmp(F.f2, j);
+                T[u++] = a * f1i * f1j + b * (f1i * f2j + f2i * f1j) + c * f2i * f2j;
+            }
+    }
+    dd8* He = reinterpret_cast<dd8*>(H + 144 * (size_t)e);
+#pragma unroll
+    for (int l = 0; l < 4; l++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const double nj = cmp(F.n, j);
+            double col[12];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const double hkj = cmp(h[k], j);
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    const double Tij = T[PK_<3>(i, j)];
+                    col[3 * k + i] = gh[k] * fma(gh[l], Tij, cmp(h[l], i) * nj) + cmp(F.n, i) * fma(gh[l], hkj, N[k][l] * nj);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 6; r++) He[6 * (3 * l + j) + r] = dd8{col[2 * r], col[2 * r + 1]};
+        }
+}
+
+// The mollified edge pairs of the same call: each 64-lane workgroup scans
+// `per` contacts, gathers the mollified ones in LDS, then one thread each
+// builds and projects the 9 x 9 matrix in the space of point differences (a
+// 9 x 9 Jacobi in registers; one wavefront per SIMD).  A kernel of its own:
+// with its registers in k_hess_api every contact would run at a quarter of
+// the occupancy, and a wavefront with one mollified lane would wait for it.
+constexpr int HM_PER = 1024;
+__global__ __launch_bounds__(64) void k_hess_moll(KParams kp, int n, int per, const double* __restrict__ x,
+                                                  const int* __restrict__ type, const double* __restrict__ dist,
+                                                  double* __restrict__ H, double* __restrict__ g, double* __restrict__ moll) {
+    __shared__ int list[HM_PER];
+    const int lane = threadIdx.x, e0 = blockIdx.x * per, e1 = min(n, e0 + per);
+    int cnt = 0;
+    for (int b = e0; b < e1; b += 64) {
+        bool on = false;
+        if (b + lane < e1) {
+            d3 P0, P1, P2, P3;
+            load_points(x, b + lane, P0, P1, P2, P3);
+            Mollifier q;
+            on = mollifier(kp.eps_x, P0, P1, P2, P3, q);
+        }
+        const unsigned long long m = __ballot(on);
+        if (on) list[cnt + __popcll(m & ((1ull << lane) - 1ull))] = b + lane;
+        cnt += __popcll(m);
     }
     __syncthreads();
-    if (kp.psd) group_psd<false>(L, lane, valid);
-    if (valid && lane < 12) {
-        for (int i = 0; i < 12; i++) H[144 * (size_t)e + 12 * lane + i] = L.H[i][lane];
-        g[12 * (size_t)e + lane] = gj;
-        if (IS_EE && lane == 0 && moll) moll[e] = mval;
+    for (int i = lane; i < cnt; i += 64) {
+        const int e = list[i];
+        d3 P0, P1, P2, P3;
+        load_points(x, e, P0, P1, P2, P3);
+        Mollifier q;
+        mollifier(kp.eps_x, P0, P1, P2, P3, q);
+        const double d = dist[e];
+        const double B0 = barrier(d, kp.d_hat, kp.kappa), B1 = barrier_d1(d, kp.d_hat, kp.kappa), B2 = barrier_d2(d, kp.d_hat, kp.kappa);
+        double K[45];
+        {
+            Frame F;
+            contact_frame(1, type[e], P0, P1, P2, P3, F);
+            mollified_matrix(F, q, B0, B1, B2, K);
+            const double gs = 2.0 * B1 * q.m * F.delta, gm = B0 * q.m1;
+            double* ge = g + 12 * (size_t)e;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    const double gx = k < 2 ? q.cn.grad(0, c) : q.cn.grad(1, c);
+                    ge[3 * k + c] = gs * F.gam[k] * cmp(F.n, c) + (k == 1 || k == 3 ? gm : -gm) * gx;
+                }
+            if (moll) moll[e] = q.m;
+        }
+        if (kp.psd) {
+            double V[81];
+            jacobi_packed<9>(K, V);
+            project_packed<9>(K, V);
+        }
+        dd8* He = reinterpret_cast<dd8*>(H + 144 * (size_t)e);
+        // entry ((k, i), (l, j)) = sum_ab Hel[a][k] K(3 a + i, 3 b + j) Hel[b][l]
+#pragma unroll
+        for (int l = 0; l < 4; l++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                double col[12];
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    double t[3], v[4];
+#pragma unroll
+                    for (int a = 0; a < 3; a++) {
+                        const double r[3] = {K[PK_<9>(3 * a + i, j)], K[PK_<9>(3 * a + i, 3 + j)], K[PK_<9>(3 * a + i, 6 + j)]};
+                        double o[4];
+                        unhelmert(r, 15u, o);
+                        t[a] = o[l];
+                    }
+                    unhelmert(t, 15u, v);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) col[3 * k + i] = v[k];
+                }
+#pragma unroll
+                for (int r = 0; r < 6; r++) He[6 * (3 * l + j) + r] = dd8{col[2 * r], col[2 * r + 1]};
+            }
     }
 }
 
@@ -765,11 +658,6 @@ __device__ __forceinline__ void load_w(const double* xbar, int id0, int id1, int
     const d3 xs[4] = {x0, x1, x2, x3};
 #pragma unroll
     for (int k = 0; k < 4; k++) { w[k][0] = 1.0; w[k][1] = xs[k].x; w[k][2] = xs[k].y; w[k][3] = xs[k].z; }
-}
-
-// Point slot k of the contact as a selector over the four points.
-__device__ __forceinline__ d3 pick(d3 p0, d3 p1, d3 p2, d3 p3, int k) {
-    return k == 0 ? p0 : (k == 1 ? p1 : (k == 2 ? p2 : p3));
 }
 
 // Class 1 contacts, one thread each: d = |r|^2, r = x_a - x_b.  In the
@@ -1154,59 +1042,6 @@ __device__ __forceinline__ void scalars_c2(const WorldArgs& a, const Stage& st, 
     stage_flush<16>(st, a.rec, REC, R_Z);
 }
 
-// packed upper-triangle index of an N x N symmetric matrix
-template <int N> __host__ __device__ constexpr int PK_(int p, int q) {
-    return p <= q ? p * N - p * (p - 1) / 2 + (q - p) : q * N - q * (q - 1) / 2 + (p - q);
-}
-// Cyclic Jacobi on a packed symmetric matrix A (registers, static indices)
-// with the eigenvectors V (row-major N x N, registers); rotations of entries
-// below JACOBI_SKIP |A|_F are skipped, and a scheduling barrier after each
-// rotation bounds the live ranges.  Returns with the eigenvalues on A's diagonal.
-template <int N>
-__device__ __forceinline__ void jacobi_packed(double (&A)[N * (N + 1) / 2], double (&V)[N * N]) {
-#pragma unroll
-    for (int e = 0; e < N * N; e++) V[e] = (e % (N + 1) == 0) ? 1.0 : 0.0;
-    for (int sweep = 0; sweep < MAX_SWEEPS; sweep++) {
-        double off = 0.0, tot = 0.0;
-#pragma unroll
-        for (int p = 0; p < N; p++)
-#pragma unroll
-            for (int q = p; q < N; q++) {
-                const double x = A[PK_<N>(p, q)] * A[PK_<N>(p, q)];
-                if (p == q) tot += x; else { off += 2.0 * x; tot += 2.0 * x; }
-            }
-        if (off <= JACOBI_TOL * tot || off == 0.0) break;
-        const double thr = JACOBI_SKIP * sqrt(tot);
-#pragma unroll
-        for (int p = 0; p < N - 1; p++)
-#pragma unroll
-            for (int q = p + 1; q < N; q++) {
-                const double apq = A[PK_<N>(p, q)];
-                if (fabs(apq) > thr) {
-                    const double app = A[PK_<N>(p, p)], aqq = A[PK_<N>(q, q)];
-                    double c, s, t;
-                    jacobi_cs(app, aqq, apq, c, s, t);
-#pragma unroll
-                    for (int k = 0; k < N; k++) {
-                        if (k == p || k == q) continue;
-                        const double akp = A[PK_<N>(k, p)], akq = A[PK_<N>(k, q)];
-                        A[PK_<N>(k, p)] = fma(c, akp, -s * akq);
-                        A[PK_<N>(k, q)] = fma(s, akp, c * akq);
-                    }
-                    A[PK_<N>(p, p)] = fma(-t, apq, app);
-                    A[PK_<N>(q, q)] = fma(t, apq, aqq);
-                    A[PK_<N>(p, q)] = 0.0;
-#pragma unroll
-                    for (int k = 0; k < N; k++) {
-                        const double vkp = V[N * k + p], vkq = V[N * k + q];
-                        V[N * k + p] = fma(c, vkp, -s * vkq);
-                        V[N * k + q] = fma(s, vkp, c * vkq);
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-    }
-}
 // PK = V diag(max(w, 0)) V^T into R[R_PK], row-major N x N
 template <int N>
 __device__ __forceinline__ void write_projection(const double (&A)[N * (N + 1) / 2], const double (&V)[N * N], double* R) {
@@ -1496,7 +1331,7 @@ extern "C" int adb_ipc_hess_pt_12x12_batched(const adb_kernel_config* cfg, int n
                                              const double* dist, double* H, double* g, void* stream) {
     if (n < 0) return ADB_E_ARG;
     if (n == 0) return ADB_OK;
-    hipLaunchKernelGGL(k_hess_api<0>, dim3((n + CPW - 1) / CPW), dim3(64), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(k_hess_api<0>, dim3((n + 63) / 64), dim3(64), 0, (hipStream_t)stream,
                        api_kp(cfg), n, pt, type, dist, H, g, (double*)nullptr);
     return hipGetLastError() == hipSuccess ? ADB_OK : ADB_E_HIP;
 }
@@ -1504,8 +1339,11 @@ extern "C" int adb_ipc_hess_ee_12x12_batched(const adb_kernel_config* cfg, int n
                                              const double* dist, double* H, double* g, double* moll, void* stream) {
     if (n < 0) return ADB_E_ARG;
     if (n == 0) return ADB_OK;
-    hipLaunchKernelGGL(k_hess_api<1>, dim3((n + CPW - 1) / CPW), dim3(64), 0, (hipStream_t)stream,
-                       api_kp(cfg), n, ee, type, dist, H, g, moll);
+    const KParams kp = api_kp(cfg);
+    hipLaunchKernelGGL(k_hess_api<1>, dim3((n + 63) / 64), dim3(64), 0, (hipStream_t)stream, kp, n, ee, type, dist, H, g, moll);
+    // about one workgroup per SIMD, at most HM_PER contacts each
+    const int per = std::min(HM_PER, std::max(64, (n / 1024 + 63) / 64 * 64));
+    hipLaunchKernelGGL(k_hess_moll, dim3((n + per - 1) / per), dim3(64), 0, (hipStream_t)stream, kp, n, per, ee, type, dist, H, g, moll);
     return hipGetLastError() == hipSuccess ? ADB_OK : ADB_E_HIP;
 }
 
