@@ -3,16 +3,24 @@
 // solve of ABD::solve (model/abd.cpp:263-291): dq = -H^{-1} g.
 //
 // Two launches per iteration, no atomics and no host round trip:
-//   spmv(k)  : every wave first sums the update partials of iteration k - 1
-//              (r.z, r.r per update workgroup) in a fixed order; from them the
-//              stop test (r.r <= rtol^2 b.b) and beta = rz_k / rz_{k-1}; then
-//              p = z + beta p_old (on the fly for every column block, written
-//              for the workgroup's own rows into the other p buffer), y = H p,
-//              and one p.y partial per workgroup
-//   update(k): every wave sums the p.y partials in a fixed order, alpha =
+//   spmv(k)  : every workgroup first sums the update partials of iteration
+//              k - 1 (r.z, r.r per update workgroup) in a fixed order; from
+//              them the stop test (r.r <= rtol^2 b.b) and beta = rz_k /
+//              rz_{k-1}; then p = z + beta p_old (on the fly for every column
+//              block, written for the workgroup's own rows into the other p
+//              buffer), y = H p, and one p.y partial per workgroup
+//   update(k): every workgroup sums the p.y partials in a fixed order, alpha =
 //              rz / pAp, x += alpha p, r -= alpha y, z = M^-1 r (explicit
 //              inverse of the diagonal block, 12 lanes per body), and one
 //              (r.z, r.r) partial per workgroup
+// At most SPMV_WGS and UPD_WGS workgroups, which loop over their rows or
+// groups: every workgroup reads every partial of the other kernel, so one
+// partial per 4 rows or per group, read by each wave, made an iteration
+// quadratic in the bodies.  27 000 bodies in 256 scenes: 305 + 97 -> 13 + 24 us
+// an iteration; 10 000 cards: 23 + 20 -> 13 + 18 us.  Small worlds are bound by
+// the chain of dependent loads, which the kernels issue in three rounds
+// ahead of the scalars: a chain of 64 tori 5.3 + 6.1 -> 4.2 + 4.9 us, of which
+// an empty launch is 1.9 us each.
 // Every workgroup evaluates the same scalars from the same partials in the
 // same order, so they agree bit for bit; once the stop test holds every kernel
 // returns at once, and the host queues iterations in batches, checking the
@@ -25,53 +33,92 @@
 namespace adb {
 
 // scalars
-enum { S_STOP = 0, S_ITERS, S_BB, S_RZ0, S_RZ1, S_COUNT };
+// (S_KBASE: iterations of the batches before this one; S_BRUN: batched worlds,
+// 1 while some scene is above its tolerance)
+enum { S_STOP = 0, S_ITERS, S_BB, S_RZ0, S_RZ1, S_KBASE, S_BRUN, S_COUNT };
 // stop flag values
 enum { RUN = 0, CONVERGED = 1, BREAKDOWN = 2, NONFINITE = 3 };
 
 constexpr int SP_ROWS = 4;       // block rows per spmv workgroup (one 64-lane team each)
+// workgroups of an spmv or update launch: all that are resident at once or
+// two rounds of them, and no more partials than one round of loads of the
+// other kernel's workgroup takes (8 per thread)
+constexpr int SPMV_WGS = 1024, UPD_WGS = 2048;
 // iterations queued between host checks: w.tune.pcg_batch (even)
 
-// fixed-order wave sum, broadcast from lane 0
+// The value of lane i ^ m (m = 32, 16, 8) or, where the lanes of a 16-lane row
+// already repeat with period 2 m, of lane i ^ m for m = 4, 2, 1: lane swaps
+// and row rotations, which stay in the vector unit.
+template <int M> __device__ __forceinline__ double add_lane_xor(double v) {
+    int2 a = *reinterpret_cast<int2*>(&v), b;
+    if constexpr (M >= 16) {
+        // both results of the swap: the lanes' own halves and the others'
+        auto lo = M == 32 ? __builtin_amdgcn_permlane32_swap(a.x, a.x, false, false) : __builtin_amdgcn_permlane16_swap(a.x, a.x, false, false);
+        auto hi = M == 32 ? __builtin_amdgcn_permlane32_swap(a.y, a.y, false, false) : __builtin_amdgcn_permlane16_swap(a.y, a.y, false, false);
+        a = make_int2(lo[0], hi[0]);
+        b = make_int2(lo[1], hi[1]);
+    } else {
+        b.x = __builtin_amdgcn_update_dpp(0, a.x, 0x120 + M, 0xf, 0xf, false);
+        b.y = __builtin_amdgcn_update_dpp(0, a.y, 0x120 + M, 0xf, 0xf, false);
+    }
+    return *reinterpret_cast<double*>(&a) + *reinterpret_cast<double*>(&b);
+}
+// fixed-order wave sum, in every lane
 __device__ __forceinline__ double wave_sum(double v) {
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_down(v, m);
-    return __shfl(v, 0);
+    v = add_lane_xor<32>(v);
+    v = add_lane_xor<16>(v);
+    v = add_lane_xor<8>(v);
+    v = add_lane_xor<4>(v);
+    v = add_lane_xor<2>(v);
+    return add_lane_xor<1>(v);
 }
-// Fixed-order sums of n values (lane l adds l, l + 64, ... in order, then
-// the wave sum).  The loads are issued 8 per lane at a time: a loop of
-// dependent adds would wait for one L2 round trip per value, which for ~1000
-// partials made up most of a PCG iteration.
-constexpr int SUM_U = 8;
-__device__ __forceinline__ double wave_sum_array(const double* v, int n) {
-    const int l = threadIdx.x % 64;
-    double s = 0.0;
-    for (int i0 = l; i0 < n; i0 += SUM_U * 64) {
-        double t[SUM_U];
-#pragma unroll
-        for (int u = 0; u < SUM_U; u++) t[u] = i0 + 64 * u < n ? v[i0 + 64 * u] : 0.0;
-#pragma unroll
-        for (int u = 0; u < SUM_U; u++)
-            if (i0 + 64 * u < n) s += t[u];
-    }
-    return wave_sum(s);
+// Value i of a wavefront's copy of an array (lane k holds value k).
+__device__ __forceinline__ double lane_value(double v, int i) {
+    const int2 a = *reinterpret_cast<int2*>(&v);
+    const int2 b = make_int2(__builtin_amdgcn_readlane(a.x, i), __builtin_amdgcn_readlane(a.y, i));
+    double r;
+    __builtin_memcpy(&r, &b, 8);
+    return r;
 }
-__device__ __forceinline__ void wave_sum_array2(const double* a, const double* b, int n, double& ra, double& rb) {
-    const int l = threadIdx.x % 64;
-    double sa = 0.0, sb = 0.0;
-    for (int i0 = l; i0 < n; i0 += SUM_U * 64) {
-        double ta[SUM_U], tb[SUM_U];
+// Fixed-order sums of n values, the same in every thread of a workgroup of T,
+// in two parts: load issues the loads, so the caller can place them among its
+// own, done adds.  Each wave sums all the values itself (lane l adds l,
+// l + 64, ... in order, then the wave sum); beyond 512 values they are split
+// over the workgroup's waves, whose sums are added in wave order behind one
+// barrier (SPLIT).  U values per lane, n <= 64 U or T U.
+template <int T, int U, bool SPLIT> struct PartSum {
+    static constexpr int NT = SPLIT ? T : 64;
+    double x[U];
+    __device__ __forceinline__ void load(const double* __restrict__ v, int n) {
+        const int t = SPLIT ? threadIdx.x : threadIdx.x % 64;
 #pragma unroll
-        for (int u = 0; u < SUM_U; u++) {
-            const bool in = i0 + 64 * u < n;
-            ta[u] = in ? a[i0 + 64 * u] : 0.0;
-            tb[u] = in ? b[i0 + 64 * u] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < SUM_U; u++)
-            if (i0 + 64 * u < n) { sa += ta[u]; sb += tb[u]; }
+        for (int u = 0; u < U; u++) x[u] = v[min(t + NT * u, n - 1)];
     }
-    ra = wave_sum(sa);
-    rb = wave_sum(sb);
+    __device__ __forceinline__ double wave(int n) const {
+        const int t = SPLIT ? threadIdx.x : threadIdx.x % 64;
+        double s = 0.0;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (t + NT * u < n) s += x[u];
+        return wave_sum(s);
+    }
+};
+// the waves' sums (SPLIT) added in wave order; one barrier, sh is not reused
+template <int T, int NV> __device__ __forceinline__ void add_waves(double (*sh)[NV], double (&v)[NV]) {
+    if (threadIdx.x % 64 == 0)
+        for (int k = 0; k < NV; k++) sh[threadIdx.x / 64][k] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+        v[k] = 0.0;
+#pragma unroll
+        for (int w = 0; w < T / 64; w++) v[k] += sh[w][k];
+    }
+}
+// orders a wave's LDS accesses among its own lanes
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 // fixed-order workgroup sum (one value per wave combined in wave order)
 __device__ double wg_sum(double v, double* sh) {
@@ -86,89 +133,110 @@ __device__ double wg_sum(double v, double* sh) {
     return r;
 }
 
-// Preconditioner application for one body group (one wave per group):
-// z = M_g^-1 r on the group's rows (n = 12 bodies <= GN), rows i = lane, lane + 64.
+// Preconditioner of the body groups: z = M_g^-1 r on group g's rows (n = 12
+// bodies <= GN); group tables hold B entries, those past *count are unused.
 constexpr int GN = 96;
 struct Groups { const int* off; const int* body; const long long* moff; const double* Minv; const int* count; };
 
-// initial: x = 0, r = -g, z = M^-1 r, p_old = 0, (r.z, r.r) partials per group
-__global__ __launch_bounds__(64) void k_pcg_init(int B, Groups G, const double* __restrict__ g, double* __restrict__ x,
-                                                 double* __restrict__ r, double* __restrict__ z, double* __restrict__ p0,
-                                                 double* __restrict__ partB, double* __restrict__ scal, int* __restrict__ kbase) {
-    __shared__ double rs[GN];
-    __shared__ int bod[GN / 12];
-    const int gi = blockIdx.x, l = threadIdx.x;
-    if (gi == 0 && l == 0) { scal[S_STOP] = RUN; scal[S_ITERS] = 0.0; *kbase = 0; }
-    if (gi >= *G.count) return;
-    const int m = G.off[gi + 1] - G.off[gi], n = 12 * m;
-    if (l < m) bod[l] = G.body[G.off[gi] + l];
-    __syncthreads();
-    for (int i = l; i < n; i += 64) {
-        const size_t k = 12 * (size_t)bod[i / 12] + i % 12;
-        const double rk = -g[k];
-        x[k] = 0.0; r[k] = rk; p0[k] = 0.0;
-        rs[i] = rk;
-    }
-    __syncthreads();
-    const double* M = G.Minv + G.moff[gi];
-    double rz = 0.0, rr = 0.0;
-    for (int i = l; i < n; i += 64) {
-        double zi = 0.0;
-        for (int j = 0; j < n; j++) zi += M[(size_t)j * n + i] * rs[j];
-        z[12 * (size_t)bod[i / 12] + i % 12] = zi;
-        rz += rs[i] * zi; rr += rs[i] * rs[i];
-    }
-    rz = wave_sum(rz);
-    rr = wave_sum(rr);
-    if (l == 0) { partB[gi] = rz; partB[B + gi] = rr; }
-}
 // Batched worlds: each scene's residual test, |r_s|^2 <= rtol^2 |b_s|^2, from
-// the group partials (groups are numbered scene by scene); first = the
-// partials of iteration 0 (|b_s|^2 = |r_s|^2 then).  One workgroup; brun = 1
-// while some scene is above its tolerance.
-__global__ __launch_bounds__(1024) void k_pcg_scene_stop(int S, int B, const int* __restrict__ sc_goff, double rtol2, int first,
-                                                         const double* __restrict__ partB, double* __restrict__ sbb,
-                                                         const double* __restrict__ scal, int* __restrict__ brun) {
+// the groups' r.r (groups are numbered scene by scene); first = those of
+// iteration 0 (|b_s|^2 = |r_s|^2 then).  One workgroup, SC_L lanes per scene,
+// loads in flight together; S_BRUN = 1 while some scene is above its tolerance.
+constexpr int SC_L = 4;
+__global__ __launch_bounds__(1024) void k_pcg_scene_stop(int S, const int* __restrict__ sc_goff, double rtol2, int first,
+                                                         const double* __restrict__ grr, double* __restrict__ sbb, double* scal) {
     __shared__ int any;
     if (threadIdx.x == 0) any = 0;
     __syncthreads();
     if (scal[S_STOP] == RUN) {
         int mine = 0;
-        for (int s = threadIdx.x; s < S; s += blockDim.x) {
+        const int l = threadIdx.x % SC_L;
+        for (int s = threadIdx.x / SC_L; s < S; s += blockDim.x / SC_L) {
+            const int e = sc_goff[s + 1];
             double rr = 0.0;
-            for (int g = sc_goff[s]; g < sc_goff[s + 1]; g++) rr += partB[B + g];
-            if (first) sbb[s] = rr;
-            if (!(rr <= rtol2 * sbb[s])) mine = 1;
+            for (int g = sc_goff[s] + l; g < e; g += 8 * SC_L) {
+                double v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = g + SC_L * u < e ? grr[g + SC_L * u] : 0.0;
+#pragma unroll
+                for (int u = 0; u < 8; u++) rr += v[u];
+            }
+            for (int m = 1; m < SC_L; m *= 2) rr += __shfl_xor(rr, m);
+            if (first && l == 0) sbb[s] = rr;
+            if (!(rr <= rtol2 * (first ? rr : sbb[s]))) mine = 1;
         }
         if (mine) any = 1;
     }
     __syncthreads();
-    if (threadIdx.x == 0) *brun = any;
+    if (threadIdx.x == 0) scal[S_BRUN] = any;
 }
 
 // iteration base of the next batch
-__global__ void k_pcg_advance(int* kbase, int n) { if (threadIdx.x == 0 && blockIdx.x == 0) *kbase += n; }
+__global__ void k_pcg_advance(double* scal, int n) { if (threadIdx.x == 0 && blockIdx.x == 0) scal[S_KBASE] += n; }
 
-__global__ __launch_bounds__(64 * SP_ROWS) void k_pcg_spmv(int B, const int* __restrict__ kbase, int kloc, double rtol2,
-                                                           const int* __restrict__ gcount,
+// A lane's share of one 12 x 12 block of a row: 12 lanes per block (lane r its
+// row r), five blocks of the row at a time.
+struct RowBlock { double H[12]; double2 z[6], p[6]; };
+__device__ __forceinline__ void load_block(RowBlock& b, int k, int col, int r, const double* __restrict__ Hval,
+                                           const double* __restrict__ z, const double* __restrict__ pold) {
+    const double* H = Hval + 144 * (size_t)k + r;
+    const size_t cb = 6 * (size_t)col;
+#pragma unroll
+    for (int c = 0; c < 12; c++) b.H[c] = H[c * 12];
+    const double2* z2 = reinterpret_cast<const double2*>(z) + cb;
+    const double2* p2 = reinterpret_cast<const double2*>(pold) + cb;
+#pragma unroll
+    for (int c = 0; c < 6; c++) { b.z[c] = z2[c]; b.p[c] = p2[c]; }
+}
+__device__ __forceinline__ double row_product(const RowBlock& b, double beta) {
+    double s = 0.0;
+#pragma unroll
+    for (int c = 0; c < 6; c++) {
+        s += b.H[2 * c] * (b.z[c].x + beta * b.p[c].x);
+        s += b.H[2 * c + 1] * (b.z[c].y + beta * b.p[c].y);
+    }
+    return s;
+}
+template <int U, bool SPLIT>
+__global__ __launch_bounds__(64 * SP_ROWS, U == 8 && !SPLIT ? 3 : 4) void k_pcg_spmv(int B, int kloc, double rtol2, int nbU, int batched,
                                                            const int* __restrict__ row_ptr,
                                                            const int* __restrict__ col_idx, const double* __restrict__ Hval,
                                                            const double* __restrict__ z, const double* __restrict__ pold,
                                                            double* __restrict__ pnew, double* __restrict__ y,
                                                            const double* __restrict__ partB, double* __restrict__ partA,
-                                                           double* __restrict__ scal, const int* __restrict__ brun) {
-    __shared__ double sh[SP_ROWS];
+                                                           double* scal) {
+    __shared__ double sh[SP_ROWS], sh2[SP_ROWS][2];
     __shared__ double acc_sh[SP_ROWS][5][12];
-    if (scal[S_STOP] != RUN) return;
-    const int iter = *kbase + kloc;
+    const int team = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const int g = lane / 12, r = lane % 12;
+    const int stride = gridDim.x * SP_ROWS;
+    int row = blockIdx.x * SP_ROWS + team;
+    // Three rounds of loads, none of which waits for the scalars: the row's
+    // extent (and the next row's), the scalars and the partials; the first
+    // block and its column; z and p_old.
+    int k0 = 0, k1 = 0;
+    if (row < B) { k0 = row_ptr[row]; k1 = row_ptr[row + 1]; }
+    int n0 = 0, n1 = 0, ncol = 0;                 // the next row's extent and first column
+    if (row + stride < B) { n0 = row_ptr[row + stride]; n1 = row_ptr[row + stride + 1]; }
+    const double sc = scal[min(lane, (int)S_COUNT - 1)];
+    PartSum<64 * SP_ROWS, U, SPLIT> prz, prr;
+    prz.load(partB, nbU);
+    prr.load(partB + nbU, nbU);
+    RowBlock blk;
+    const bool first = g < 5 && k0 + g < k1;
+    if (first) load_block(blk, k0 + g, col_idx[k0 + g], r, Hval, z, pold);
+    double2 zo = make_double2(0.0, 0.0);          // the row's own z and p_old
+    if (row < B && lane < 12) zo = make_double2(z[12 * (size_t)row + lane], pold[12 * (size_t)row + lane]);
+    if (lane_value(sc, S_STOP) != RUN) return;
     // scalars of iteration iter - 1 (identical in every wave of every workgroup)
-    const int nbU = *gcount;
-    double RZ, RR;
-    wave_sum_array2(partB, partB + B, nbU, RZ, RR);
-    const double bb = iter == 0 ? RR : scal[S_BB];
+    const int iter = (int)lane_value(sc, S_KBASE) + kloc;
+    double rzr[2] = {prz.wave(nbU), prr.wave(nbU)};
+    if (SPLIT) add_waves<64 * SP_ROWS>(sh2, rzr);
+    const double RZ = rzr[0], RR = rzr[1];
+    const double bb = iter == 0 ? RR : lane_value(sc, S_BB);
     int stop = RUN;
     if (!std::isfinite(RR) || !std::isfinite(RZ)) stop = NONFINITE;
-    else if (brun ? *brun == 0 : RR <= rtol2 * bb) stop = CONVERGED;   // batched: every scene's own test
+    else if (batched ? lane_value(sc, S_BRUN) == 0.0 : RR <= rtol2 * bb) stop = CONVERGED;   // batched: every scene's own test
     else if (!(RZ > 0.0)) stop = BREAKDOWN;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (iter == 0) scal[S_BB] = RR;
@@ -176,104 +244,159 @@ __global__ __launch_bounds__(64 * SP_ROWS) void k_pcg_spmv(int B, const int* __r
         if (stop != RUN) { scal[S_STOP] = stop; scal[S_ITERS] = iter; }
     }
     if (stop != RUN) return;
-    const double beta = iter == 0 ? 0.0 : RZ / scal[S_RZ0 + ((iter - 1) & 1)];
-    const int team = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int row = blockIdx.x * SP_ROWS + team;
-    const int g = lane / 12, r = lane % 12;
-    if (row < B && g < 5) {
-        double acc = 0.0;
-        for (int k = row_ptr[row] + g; k < row_ptr[row + 1]; k += 5) {
-            const double* H = Hval + 144 * (size_t)k;
-            const size_t cb = 12 * (size_t)col_idx[k];
-            double s = 0.0;
-#pragma unroll
-            for (int c = 0; c < 12; c++) s += H[c * 12 + r] * (z[cb + c] + beta * pold[cb + c]);
-            acc += s;
-        }
-        acc_sh[team][g][r] = acc;
-    }
-    __syncthreads();
+    const double beta = iter == 0 ? 0.0 : RZ / lane_value(sc, S_RZ0 + ((iter - 1) & 1));
     double prod = 0.0;
-    if (row < B && lane < 12) {
-        const size_t k = 12 * (size_t)row + lane;
-        const double yr = (((acc_sh[team][0][lane] + acc_sh[team][1][lane]) + acc_sh[team][2][lane]) + acc_sh[team][3][lane]) +
-                          acc_sh[team][4][lane];
-        const double pr = z[k] + beta * pold[k];
-        y[k] = yr;
-        pnew[k] = pr;
-        prod = pr * yr;
+    while (row < B) {
+        if (g < 5 && n0 + g < n1) ncol = col_idx[n0 + g];
+        if (g < 5) {
+            double acc = 0.0;
+            if (k0 + g < k1) acc += row_product(blk, beta);
+            for (int k = k0 + g + 5; k < k1; k += 5) {
+                load_block(blk, k, col_idx[k], r, Hval, z, pold);
+                acc += row_product(blk, beta);
+            }
+            acc_sh[team][g][r] = acc;
+        }
+        wave_fence();       // a row belongs to one wave
+        if (lane < 12) {
+            const size_t k = 12 * (size_t)row + lane;
+            const double yr = (((acc_sh[team][0][lane] + acc_sh[team][1][lane]) + acc_sh[team][2][lane]) + acc_sh[team][3][lane]) +
+                              acc_sh[team][4][lane];
+            const double pr = zo.x + beta * zo.y;
+            y[k] = yr;
+            pnew[k] = pr;
+            prod += pr * yr;
+        }
+        wave_fence();
+        row += stride;
+        if (row >= B) break;
+        k0 = n0; k1 = n1;
+        if (g < 5 && k0 + g < k1) load_block(blk, k0 + g, ncol, r, Hval, z, pold);
+        if (lane < 12) zo = make_double2(z[12 * (size_t)row + lane], pold[12 * (size_t)row + lane]);
+        n0 = n1 = 0;
+        if (row + stride < B) { n0 = row_ptr[row + stride]; n1 = row_ptr[row + stride + 1]; }
     }
     prod = wg_sum(prod, sh);
     if (threadIdx.x == 0) partA[blockIdx.x] = prod;
 }
 
 // UPD_T lanes per group: row i = t % GN of the group, column half t / GN of
-// z = M^-1 r, the two halves combined in order
-constexpr int UPD_T = 2 * GN;
-__global__ __launch_bounds__(UPD_T) void k_pcg_update(int B, const int* __restrict__ kbase, int kloc, int nbS, Groups G,
-                                                      const double* __restrict__ p, const double* __restrict__ y,
+// z = M^-1 r, the two halves combined in order; groups gi = blockIdx.x,
+// + gridDim.x, ....  FIRST: x = 0, r = -g, p_old = 0 (y = the gradient, p
+// written) instead of the update of x and r by alpha, and the scalars of a
+// new solve.  The loads are issued in three rounds again: group table,
+// scalars and partials; body and the lane's part of the inverse (48 values in
+// flight); the vectors.
+constexpr int UPD_T = 2 * GN, GH = GN / 2;
+struct GroupRow { double M[GH]; size_t k; int m, j0; bool on; };      // k: the row's element; columns [j0, j0 + 6 m)
+__device__ __forceinline__ void load_group(GroupRow& q, const Groups& G, int gi, int t) {
+    const int cnt = *G.count, o0 = G.off[gi], o1 = G.off[gi + 1];
+    const double* M = G.Minv + G.moff[gi];
+    const int i = t % GN, h = t / GN;
+    q.m = gi < cnt ? o1 - o0 : 0;
+    q.on = i < 12 * q.m;
+    q.j0 = h * 6 * q.m;
+    q.k = 0;
+    if (!q.on) return;
+    q.k = 12 * (size_t)G.body[o0 + i / 12] + i % 12;
+    M += (size_t)q.j0 * (12 * q.m) + i;
+#pragma unroll
+    for (int s = 0; s < GN / 12; s++)
+        if (s < q.m) {
+#pragma unroll
+            for (int u = 6 * s; u < 6 * s + 6; u++) q.M[u] = M[u * 12 * q.m];
+        }
+}
+template <bool FIRST, int U, bool SPLIT>
+__global__ __launch_bounds__(UPD_T) void k_pcg_update(int kloc, int nbS, Groups G,
+                                                      double* __restrict__ p, const double* __restrict__ y,
                                                       double* __restrict__ x, double* __restrict__ r, double* __restrict__ z,
                                                       const double* __restrict__ partA, double* __restrict__ partB,
-                                                      double* __restrict__ scal) {
+                                                      double* __restrict__ grr, double* scal) {
     __shared__ double rs[GN];
     __shared__ double half2[GN];
-    __shared__ double red[UPD_T / 64][2];
-    __shared__ int bod[GN / 12];
-    if (scal[S_STOP] != RUN) return;
-    const int gi = blockIdx.x, t = threadIdx.x;
-    if (gi > 0 && gi >= *G.count) return;     // workgroup 0 also reports a breakdown
-    const int iter = *kbase + kloc;
-    const double pAp = wave_sum_array(partA, nbS);
-    const double RZ = scal[S_RZ0 + (iter & 1)];
-    if (!(pAp > 0.0) || !std::isfinite(pAp)) {
-        if (gi == 0 && t == 0) { scal[S_STOP] = std::isfinite(pAp) ? BREAKDOWN : NONFINITE; scal[S_ITERS] = iter; }
-        return;
+    __shared__ double red[UPD_T / 64][2], sh1[UPD_T / 64][1];
+    const int t = threadIdx.x;
+    double sc = 0.0;
+    PartSum<UPD_T, U, SPLIT> pa;
+    if (!FIRST) {
+        sc = scal[min(t % 64, (int)S_COUNT - 1)];
+        pa.load(partA, nbS);
     }
-    if (gi >= *G.count) return;
-    const double alpha = RZ / pAp;
-    const int m = G.off[gi + 1] - G.off[gi], n = 12 * m;
-    if (t < m) bod[t] = G.body[G.off[gi] + t];
-    __syncthreads();
-    if (t < n) {
-        const size_t k = 12 * (size_t)bod[t / 12] + t % 12;
-        x[k] += alpha * p[k];
-        const double rk = r[k] - alpha * y[k];
-        r[k] = rk;
-        rs[t] = rk;
+    const int ng = *G.count;
+    GroupRow q;
+    load_group(q, G, blockIdx.x, t);
+    const bool vec = t < GN;
+    double xk = 0.0, pk = 0.0, yk = 0.0, rk = 0.0;
+    if (q.on && vec) {
+        yk = y[q.k];
+        if (!FIRST) { xk = x[q.k]; pk = p[q.k]; rk = r[q.k]; }
     }
-    __syncthreads();
-    const double* M = G.Minv + G.moff[gi];
-    const int i = t % GN, h = t / GN, j0 = h * ((n + 1) / 2), j1 = h ? n : (n + 1) / 2;
-    double zi = 0.0;
-    if (i < n) {
-        // loads SUM_U at a time, products added in order of j
-        int j = j0;
-        for (; j + SUM_U <= j1; j += SUM_U) {
-            double m[SUM_U];
-#pragma unroll
-            for (int u = 0; u < SUM_U; u++) m[u] = M[(size_t)(j + u) * n + i];
-#pragma unroll
-            for (int u = 0; u < SUM_U; u++) zi += m[u] * rs[j + u];
+    double alpha = 0.0;
+    if (FIRST) {
+        if (blockIdx.x == 0 && t == 0) { scal[S_STOP] = RUN; scal[S_ITERS] = 0.0; scal[S_KBASE] = 0.0; }
+    } else {
+        if (lane_value(sc, S_STOP) != RUN) return;
+        const int iter = (int)lane_value(sc, S_KBASE) + kloc;
+        double s1[1] = {pa.wave(nbS)};
+        if (SPLIT) add_waves<UPD_T>(sh1, s1);
+        const double pAp = s1[0];
+        if (!(pAp > 0.0) || !std::isfinite(pAp)) {
+            if (blockIdx.x == 0 && t == 0) { scal[S_STOP] = std::isfinite(pAp) ? BREAKDOWN : NONFINITE; scal[S_ITERS] = iter; }
+            return;
         }
-        for (; j < j1; j++) zi += M[(size_t)j * n + i] * rs[j];
+        alpha = lane_value(sc, S_RZ0 + (iter & 1)) / pAp;
     }
-    if (h == 1 && i < n) half2[i] = zi;
-    __syncthreads();
-    double rz = 0.0, rr = 0.0;
-    if (h == 0 && i < n) {
-        zi += half2[i];
-        z[12 * (size_t)bod[i / 12] + i % 12] = zi;
-        rz = rs[i] * zi; rr = rs[i] * rs[i];
+    double a0 = 0.0, a1 = 0.0;
+    for (int gi = blockIdx.x; gi < ng;) {
+        if (q.on && vec) {
+            x[q.k] = FIRST ? 0.0 : xk + alpha * pk;
+            rk = FIRST ? -yk : rk - alpha * yk;
+            if (FIRST) p[q.k] = 0.0;
+            r[q.k] = rk;
+            rs[t] = rk;
+        }
+        __syncthreads();
+        const int i = t % GN;
+        double zi = 0.0;
+        if (q.on) {
+#pragma unroll
+            for (int s = 0; s < GN / 12; s++)
+                if (s < q.m) {
+#pragma unroll
+                    for (int u = 6 * s; u < 6 * s + 6; u++) zi += q.M[u] * rs[q.j0 + u];
+                }
+        }
+        if (!vec && q.on) half2[i] = zi;
+        __syncthreads();
+        double pz = 0.0, pr = 0.0;
+        if (vec && q.on) {
+            zi += half2[i];
+            z[q.k] = zi;
+            pz = rk * zi; pr = rk * rk;
+        }
+        // the next group's loads run under the sums
+        const int gj = gi + gridDim.x;
+        if (gj < ng) {
+            load_group(q, G, gj, t);
+            if (q.on && vec) {
+                yk = y[q.k];
+                if (!FIRST) { xk = x[q.k]; pk = p[q.k]; rk = r[q.k]; }
+            }
+        }
+        pz = wave_sum(pz);
+        pr = wave_sum(pr);
+        if (t % 64 == 0) { red[t / 64][0] = pz; red[t / 64][1] = pr; }
+        __syncthreads();
+        if (t == 0) {
+            double b0 = 0.0, b1 = 0.0;
+            for (int w = 0; w < UPD_T / 64; w++) { b0 += red[w][0]; b1 += red[w][1]; }
+            a0 += b0; a1 += b1;
+            if (grr) grr[gi] = b1;
+        }
+        gi = gj;
     }
-    rz = wave_sum(rz);
-    rr = wave_sum(rr);
-    if (t % 64 == 0) { red[t / 64][0] = rz; red[t / 64][1] = rr; }
-    __syncthreads();
-    if (t == 0) {
-        double a0 = 0.0, a1 = 0.0;
-        for (int w = 0; w < UPD_T / 64; w++) { a0 += red[w][0]; a1 += red[w][1]; }
-        partB[gi] = a0; partB[B + gi] = a1;
-    }
+    if (t == 0) { partB[blockIdx.x] = a0; partB[gridDim.x + blockIdx.x] = a1; }
 }
 
 static Groups groups_of(World& w) {
@@ -282,58 +405,77 @@ static Groups groups_of(World& w) {
     return G;
 }
 
+static int spmv_wgs(int B) { return std::min((B + SP_ROWS - 1) / SP_ROWS, SPMV_WGS); }
+static int update_wgs(int B) { return std::min(B, UPD_WGS); }         // at most B groups; their count stays on the device
+
+// kernel k of a batch; the partial counts, so the sums' forms, depend on B only
+static void launch_spmv(World& w, int k, const double* pold, double* pnew) {
+    const int B = w.B, nbS = spmv_wgs(B), nbU = update_wgs(B);
+    double* partA = w.partial.p;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nbS), dim3(64 * SP_ROWS), 0, w.stream, B, k, w.P.pcg_rtol * w.P.pcg_rtol, nbU, (int)(w.S > 1),
+                           w.row_ptr.p, w.col_idx.p, w.Hval.p, w.pcg_z.p, pold, pnew, w.pcg_Ap.p, partA + nbS, partA, w.scal.p);
+    };
+    if (nbU <= 64) go(k_pcg_spmv<1, false>);
+    else if (nbU <= 512) go(k_pcg_spmv<8, false>);
+    else go(k_pcg_spmv<8, true>);
+}
+template <bool FIRST> static void launch_update(World& w, int k, double* p, const double* y) {
+    const int B = w.B, nbS = spmv_wgs(B), nbU = update_wgs(B);
+    double* partA = w.partial.p;
+    double* partB = partA + nbS;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nbU), dim3(UPD_T), 0, w.stream, k, nbS, groups_of(w), p, y, w.pcg_xo, w.pcg_r.p, w.pcg_z.p,
+                           partA, partB, w.S > 1 ? partB + 2 * nbU : (double*)nullptr, w.scal.p);
+    };
+    if (FIRST || nbS <= 64) go(k_pcg_update<FIRST, 1, false>);
+    else if (nbS <= 512) go(k_pcg_update<FIRST, 8, false>);
+    else go(k_pcg_update<FIRST, 8, true>);
+}
+static void launch_scene_stop(World& w, int first) {
+    const double* grr = w.partial.p + spmv_wgs(w.B) + 2 * update_wgs(w.B);
+    hipLaunchKernelGGL(k_pcg_scene_stop, dim3(1), dim3(1024), 0, w.stream, w.S, w.sc_goff.p, w.P.pcg_rtol * w.P.pcg_rtol, first, grr,
+                       w.pcg_sbb.p, w.scal.p);
+}
+
 // One batch = pcg_batch iterations; kernel k of the batch computes iteration
-// *kbase + k, and the last node advances *kbase.  Because the batch is even, the
+// S_KBASE + k, and the last node advances S_KBASE.  Because the batch is even, the
 // p-buffer parity of local iteration k is k & 1 in every batch, so one
 // captured graph serves every batch.
 static void enqueue_batch(World& w, int nb, bool prof) {
-    const int B = w.B;
-    const int nbS = (B + SP_ROWS - 1) / SP_ROWS;
-    const double rtol2 = w.P.pcg_rtol * w.P.pcg_rtol;
-    double* partA = w.partial.p;
-    double* partB = w.partial.p + nbS;
-    const Groups G = groups_of(w);
     double* pb[2] = {w.pcg_p.p, w.pcg_p2.p};
     for (int k = 0; k < nb; k++) {
         {
             // H blocks, their column indices, z and p_old read, p_new and y written
-            ProfScope ps(w, PK_SPMV, prof ? 1152.0 * w.nnzb + 4.0 * w.nnzb + 4.0 * 96.0 * B : 0.0);
-            hipLaunchKernelGGL(k_pcg_spmv, dim3(nbS), dim3(64 * SP_ROWS), 0, w.stream, B, w.pcg_k.p, k, rtol2, w.grp_n, w.row_ptr.p,
-                               w.col_idx.p, w.Hval.p, w.pcg_z.p, pb[k & 1], pb[(k & 1) ^ 1], w.pcg_Ap.p, partB, partA, w.scal.p,
-                               w.S > 1 ? (const int*)w.pcg_brun.p : (const int*)nullptr);
+            ProfScope ps(w, PK_SPMV, prof ? 1152.0 * w.nnzb + 4.0 * w.nnzb + 4.0 * 96.0 * w.B : 0.0);
+            launch_spmv(w, k, pb[k & 1], pb[(k & 1) ^ 1]);
         }
         {
             // group inverses read; p, y read; x, r read and written; z written
-            ProfScope ps(w, PK_PCG_UPDATE, prof ? 8.0 * (double)w.h_grp_moff.back() + 7.0 * 96.0 * B : 0.0);
-            hipLaunchKernelGGL(k_pcg_update, dim3(B), dim3(UPD_T), 0, w.stream, B, w.pcg_k.p, k, nbS, G, pb[(k & 1) ^ 1],
-                               w.pcg_Ap.p, w.pcg_xo, w.pcg_r.p, w.pcg_z.p, partA, partB, w.scal.p);
+            ProfScope ps(w, PK_PCG_UPDATE, prof ? 8.0 * (double)w.h_grp_moff.back() + 7.0 * 96.0 * w.B : 0.0);
+            launch_update<false>(w, k, pb[(k & 1) ^ 1], w.pcg_Ap.p);
         }
-        if (w.S > 1)
-            hipLaunchKernelGGL(k_pcg_scene_stop, dim3(1), dim3(1024), 0, w.stream, w.S, B, w.sc_goff.p, rtol2, 0, partB, w.pcg_sbb.p,
-                               w.scal.p, w.pcg_brun.p);
+        if (w.S > 1) launch_scene_stop(w, 0);
     }
-    hipLaunchKernelGGL(k_pcg_advance, dim3(1), dim3(64), 0, w.stream, w.pcg_k.p, nb);
+    hipLaunchKernelGGL(k_pcg_advance, dim3(1), dim3(64), 0, w.stream, w.scal.p, nb);
 }
 
 int pcg_solve(World& w, double* dq_out, int* iters, const std::function<void()>& after, bool* after_valid) {
     if (after_valid) *after_valid = false;
     const int B = w.B, n = 12 * B;
-    const int nbS = (B + SP_ROWS - 1) / SP_ROWS;
+    const int nbS = spmv_wgs(B), nbU = update_wgs(B);
     // the iterate x lives in the caller's output (12 B doubles)
     w.pcg_xo = dq_out;
     w.pcg_r.reserve(n); w.pcg_z.reserve(n); w.pcg_p.reserve(n); w.pcg_p2.reserve(n); w.pcg_Ap.reserve(n);
-    w.partial.reserve((size_t)nbS + 2 * (size_t)B); w.scal.reserve(S_COUNT); w.pcg_k.reserve(1);
-    double* partB = w.partial.p + nbS;
+    w.partial.reserve((size_t)nbS + 2 * (size_t)nbU + (w.S > 1 ? (size_t)B : 0)); w.scal.reserve(S_COUNT);
     if (!w.h_scal) ADB_HIP(hipHostMalloc((void**)&w.h_scal, 2 * S_COUNT * sizeof(double), hipHostMallocDefault));
     for (hipEvent_t& e : w.pcg_ev)
         if (!e) ADB_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    hipLaunchKernelGGL(k_pcg_init, dim3(B), dim3(64), 0, w.stream, B, groups_of(w), w.grad.p, w.pcg_xo, w.pcg_r.p, w.pcg_z.p,
-                       w.pcg_p.p, partB, w.scal.p, w.pcg_k.p);
+    if (w.S > 1) w.pcg_sbb.reserve(w.S);
+    launch_update<true>(w, 0, w.pcg_p.p, w.grad.p);
     ADB_HIP(hipGetLastError());
     if (w.S > 1) {
-        w.pcg_sbb.reserve(w.S); w.pcg_brun.reserve(1);
-        hipLaunchKernelGGL(k_pcg_scene_stop, dim3(1), dim3(1024), 0, w.stream, w.S, B, w.sc_goff.p,
-                           w.P.pcg_rtol * w.P.pcg_rtol, 1, partB, w.pcg_sbb.p, w.scal.p, w.pcg_brun.p);
+        launch_scene_stop(w, 1);
         ADB_HIP(hipGetLastError());
     }
     // the batch graph is captured once per set of buffer addresses (not while
@@ -342,8 +484,8 @@ int pcg_solve(World& w, double* dq_out, int* iters, const std::function<void()>&
     const bool use_graph = !w.prof.on && w.use_graphs;
     if (use_graph) {
         const void* key[] = {w.row_ptr.p, w.col_idx.p, w.Hval.p, w.Ginv.p, w.pcg_xo, w.pcg_r.p, w.pcg_z.p, w.pcg_p.p,
-                             w.pcg_p2.p, w.pcg_Ap.p, w.partial.p, w.scal.p, w.pcg_k.p, w.grp_off, w.grp_body, w.grp_moff,
-                             w.grp_n, w.sc_goff.p, w.pcg_sbb.p, w.pcg_brun.p};
+                             w.pcg_p2.p, w.pcg_Ap.p, w.partial.p, w.scal.p, w.grp_off, w.grp_body, w.grp_moff,
+                             w.grp_n, w.sc_goff.p, w.pcg_sbb.p};
         static_assert(sizeof key / sizeof key[0] == World::PCG_GRAPH_KEYS, "graph key size");
         const int BATCH = w.tune.pcg_batch;
         bool same = w.pcg_graph != nullptr && w.pcg_graph_batch == BATCH;
@@ -369,11 +511,7 @@ int pcg_solve(World& w, double* dq_out, int* iters, const std::function<void()>&
     // iteration's spmv, which the next batch's first spmv repeats identically
     // (same iteration, same p-buffer parity: batches are even)
     auto stop_test = [&]() {
-        const double rtol2 = w.P.pcg_rtol * w.P.pcg_rtol;
-        double* partA = w.partial.p;
-        hipLaunchKernelGGL(k_pcg_spmv, dim3(nbS), dim3(64 * SP_ROWS), 0, w.stream, B, w.pcg_k.p, 0, rtol2, w.grp_n, w.row_ptr.p,
-                           w.col_idx.p, w.Hval.p, w.pcg_z.p, w.pcg_p.p, w.pcg_p2.p, w.pcg_Ap.p, partB, partA, w.scal.p,
-                           w.S > 1 ? (const int*)w.pcg_brun.p : (const int*)nullptr);
+        launch_spmv(w, 0, w.pcg_p.p, w.pcg_p2.p);
         ADB_HIP(hipGetLastError());
     };
     // Near the iteration count of the previous solve (Newton steps change the

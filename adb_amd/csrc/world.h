@@ -217,7 +217,6 @@ struct World {
     // ---- PCG
     DBuf<double> pcg_r, pcg_z, pcg_p, pcg_p2, pcg_Ap, partial, scal;
     double* pcg_xo = nullptr;        // the solve's iterate: the caller's output buffer
-    DBuf<int> pcg_k;                 // iteration base of the queued PCG batch
     int pcg_prev_its = 0;            // iterations of the previous solve
     int* h_pairs = nullptr;          // pinned host copy of the pair count and lists (lo, hi, start)
     size_t h_pairs_cap = 0;
@@ -227,7 +226,7 @@ struct World {
     hipEvent_t ev_phase[2] = {nullptr, nullptr};   // contact terms + assembly on the stream: start, end
     bool use_graphs = true;          // ADB_PCG_GRAPH=0 turns graph capture off
     hipGraphExec_t pcg_graph = nullptr;   // one captured PCG batch
-    static constexpr int PCG_GRAPH_KEYS = 20;
+    static constexpr int PCG_GRAPH_KEYS = 18;
     const void* pcg_graph_key[PCG_GRAPH_KEYS] = {};   // buffer addresses the graph was captured with
     double* h_scal = nullptr;        // pinned host copies of the PCG scalars (2 x 8)
     hipEvent_t pcg_ev[2] = {nullptr, nullptr};
@@ -254,7 +253,6 @@ struct World {
     DBuf<int> sc_goff;                    // per scene: first preconditioner group (S + 1)
     std::vector<int> h_sc_goff;
     DBuf<double> pcg_sbb;                 // per scene: |b|^2 of the current solve
-    DBuf<int> pcg_brun;                   // 1 while some scene's residual is above its tolerance
     double* h_sred = nullptr;             // pinned host copy of sred
     std::vector<int> h_stall_pt, h_stall_vg;
     // per-scene results of the last step
