@@ -794,6 +794,8 @@ __global__ __launch_bounds__(256) void k_group_inv(const int* __restrict__ list,
 // most GMAX bodies, so the strongest couplings land inside the inverted
 // diagonal sub-matrices; every connected component of at most GMAX bodies
 // ends up as one group (the preconditioned system then decouples exactly).
+// Components of more than TREE_MIN bodies whose elimination fills in little
+// are one group too, with the factors of tree.h.
 // The pair lists go to pinned host memory before the assembly reduction is
 // queued (groups_fetch), so the host builds the groups while it runs.
 // h_pairs = [pair count, npb pair_lo, npb pair_hi, npb + 1 pair_start]: the
@@ -823,6 +825,77 @@ static void groups_fetch(World& w, int npb, const int* npd, const int* pack, hip
     }
     ADB_HIP(hipEventRecord(w.ev_pairs, st));
 }
+// The components of the contact graph of more than TREE_MIN bodies that become one
+// group each (tree.h): hg_tree (a body's component or -1), its table's offset
+// and block count, and h_tree = the group ids (filled by build_groups), then
+// the tables.  Static bodies take no part: their rows have no off-diagonal
+// blocks.
+static void plan_trees(World& w, int np, const int* plo, const int* phi) {
+    const int B = w.B;
+    std::vector<int>&par = w.hg_cpar, &tree = w.hg_tree, &loc = w.hg_loc;
+    tree.assign(B, -1);
+    w.hg_tree_tab.clear(); w.hg_tree_ne.clear(); w.h_tree.clear();
+    w.n_trees = 0;
+    // a caller that caps the iterations at a few asks for the truncated solve
+    // (and the report that it was), whose iterates are those of the small groups
+    if (w.P.pcg_max_iter < TREE_MIN_ITER) return;
+    par.resize(B);
+    for (int b = 0; b < B; b++) par[b] = b;
+    auto find = [&](int x) { while (par[x] != x) { par[x] = par[par[x]]; x = par[x]; } return x; };
+    auto coupled = [&](int p) { return w.h_mass[plo[p]] > 0.0 && w.h_mass[phi[p]] > 0.0; };
+    std::vector<int>& cnt = w.hg_ccnt;
+    cnt.assign(B, 1);
+    int big = 0;
+    for (int p = 0; p < np; p++) {
+        if (!coupled(p)) continue;
+        int a = find(plo[p]), b = find(phi[p]);
+        if (a == b) continue;
+        if (a > b) std::swap(a, b);
+        par[b] = a; cnt[a] += cnt[b];
+        big = std::max(big, cnt[a]);
+    }
+    if (big <= TREE_MIN) return;
+    // candidate components numbered by their smallest body; their bodies and pairs
+    std::vector<int>&cid = w.hg_cid, &boff = w.hg_boff, &bods = w.hg_bods, &poff = w.hg_poff, &prs = w.hg_prs;
+    cid.assign(B, -1);
+    loc.resize(B);
+    boff.assign(1, 0);
+    for (int b = 0; b < B; b++)
+        if (par[b] == b && cnt[b] > TREE_MIN && cnt[b] <= TREE_MAX) { cid[b] = (int)boff.size() - 1; boff.push_back(boff.back() + cnt[b]); }
+    const int nc = (int)boff.size() - 1;
+    bods.resize(boff.back());
+    std::vector<int>& fill = w.hg_fill;
+    fill.assign(boff.begin(), boff.end());
+    for (int b = 0; b < B; b++) {
+        const int c = cid[find(b)];
+        if (c < 0) continue;
+        cid[b] = c;                       // (the root keeps its own number)
+        loc[b] = fill[c] - boff[c];
+        bods[fill[c]++] = b;
+    }
+    poff.assign(nc + 1, 0);
+    for (int p = 0; p < np; p++)
+        if (coupled(p) && cid[plo[p]] >= 0) poff[cid[plo[p]] + 1]++;
+    for (int c = 0; c < nc; c++) poff[c + 1] += poff[c];
+    prs.resize(poff.back());
+    fill.assign(poff.begin(), poff.end());
+    for (int p = 0; p < np; p++)
+        if (coupled(p) && cid[plo[p]] >= 0) prs[fill[cid[plo[p]]]++] = p;
+    std::vector<int>& tabs = w.hg_tabs;
+    tabs.clear();
+    for (int c = 0; c < nc; c++) {
+        const int n = boff[c + 1] - boff[c], at = (int)tabs.size();
+        w.tree_plan.start(n);
+        for (int x = poff[c]; x < poff[c + 1]; x++) w.tree_plan.edge(loc[plo[prs[x]]], loc[phi[prs[x]]], 2 * prs[x]);
+        if (!w.tree_plan.finish(n, &bods[boff[c]], tabs)) continue;
+        for (int x = boff[c]; x < boff[c + 1]; x++) tree[bods[x]] = w.n_trees;
+        w.hg_tree_tab.push_back(at);
+        w.hg_tree_ne.push_back(tabs[at + 2]);
+        w.n_trees++;
+    }
+    w.h_tree.assign(w.n_trees, 0);
+    w.h_tree.insert(w.h_tree.end(), tabs.begin(), tabs.end());
+}
 static void build_groups(World& w) {
     wait_event(w, w.ev_pairs);
     const int B = w.B, npb = w.h_pairs_n, np = w.h_pairs[0];
@@ -848,9 +921,13 @@ static void build_groups(World& w) {
     size.assign(B, 1);
     for (int b = 0; b < B; b++) parent[b] = b;
     auto find = [&](int x) { while (parent[x] != x) { parent[x] = parent[parent[x]]; x = parent[x]; } return x; };
+    plan_trees(w, np, plo, phi);
+    const std::vector<int>& tree = w.hg_tree;      // a body's tree component, -1: none
     for (int p : order) {
         int ra = find(plo[p]), rb = find(phi[p]);
-        if (ra == rb || size[ra] + size[rb] > GMAX) continue;
+        if (ra == rb) continue;
+        const int ta = tree[plo[p]], tb = tree[phi[p]];
+        if (ta != tb || (ta < 0 && size[ra] + size[rb] > GMAX)) continue;
         if (ra > rb) std::swap(ra, rb);
         parent[rb] = ra; size[ra] += size[rb];
     }
@@ -876,7 +953,9 @@ static void build_groups(World& w) {
     w.h_grp_moff[0] = 0;
     for (int g = 0; g < G; g++) {
         const long long n = 12 * (long long)(w.h_grp_off[g + 1] - w.h_grp_off[g]);
-        w.h_grp_moff[g + 1] = w.h_grp_moff[g] + n * n;
+        const int tr = tree[w.h_grp_body[w.h_grp_off[g]]];
+        w.h_grp_moff[g + 1] = w.h_grp_moff[g] + (tr < 0 ? n * n : TreePlan::doubles((int)(n / 12), w.hg_tree_ne[tr]));
+        if (tr >= 0) w.h_tree[tr] = g;
     }
     w.n_groups = G;
     if (w.S > 1) {
@@ -896,7 +975,10 @@ static void build_groups(World& w) {
     // the inverse kernel gives each class its own team width): 5..GMAX
     // bodies, 2..4, single bodies
     w.h_glist.clear();
-    for (int g = 0; g < w.n_groups; g++) if (w.h_grp_off[g + 1] - w.h_grp_off[g] > 4) w.h_glist.push_back(g);
+    for (int g = 0; g < w.n_groups; g++) {
+        const int m = w.h_grp_off[g + 1] - w.h_grp_off[g];
+        if (m > 4 && m <= GMAX) w.h_glist.push_back(g);
+    }
     w.n_glist[0] = (int)w.h_glist.size();
     for (int g = 0; g < w.n_groups; g++) {
         const int m = w.h_grp_off[g + 1] - w.h_grp_off[g];
@@ -909,7 +991,7 @@ static void build_groups(World& w) {
     // it has completed before it is rewritten).  Offsets depend on B only (at
     // most B groups), so the tables' device addresses stay the same from one
     // Newton iteration to the next (the captured PCG batch is keyed on them).
-    const size_t nll = (size_t)B + 1, nint = (size_t)(B + 1) + B + B + 1, total = nll + (nint + 1) / 2;
+    const size_t nll = (size_t)B + 1, nint = (size_t)(B + 1) + B + B + B + 1, total = nll + (nint + 1) / 2;
     if (!w.ev_grp) ADB_HIP(hipEventCreateWithFlags(&w.ev_grp, hipEventDisableTiming));
     wait_event(w, w.ev_grp);
     if (total > w.h_grp_pack_cap) {
@@ -925,15 +1007,34 @@ static void build_groups(World& w) {
         std::memcpy(hm, w.h_grp_moff.data(), (size_t)(G + 1) * sizeof(long long));
         std::memcpy(hi, w.h_grp_off.data(), (size_t)(G + 1) * sizeof(int));
         std::memcpy(hi + B + 1, w.h_grp_body.data(), (size_t)B * sizeof(int));
-        std::memcpy(hi + 2 * B + 1, w.h_glist.data(), (size_t)G * sizeof(int));
-        hi[3 * B + 1] = G;
+        std::memcpy(hi + 2 * B + 1, w.h_glist.data(), w.h_glist.size() * sizeof(int));
+        int* ht = hi + 3 * B + 1;
+        for (int g = 0; g < G; g++) {
+            const int tr = tree[w.h_grp_body[w.h_grp_off[g]]];
+            ht[g] = tr < 0 ? -1 : w.hg_tree_tab[tr];
+        }
+        hi[4 * B + 1] = G;
     }
     w.grp_moff = w.grp_pack.p;
     w.grp_off = reinterpret_cast<int*>(w.grp_pack.p + nll);
     w.grp_body = w.grp_off + B + 1;
     w.glist = w.grp_body + B;
-    w.grp_n = w.glist + B;
+    w.grp_tree = w.glist + B;
+    w.grp_n = w.grp_tree + B;
     ADB_HIP(hipMemcpyAsync(w.grp_pack.p, w.h_grp_pack, total * sizeof(long long), hipMemcpyHostToDevice, w.stream));
+    if (w.n_trees > 0) {
+        // the tree groups' ids, then their tables
+        const size_t nt = w.h_tree.size();
+        if (nt > w.h_tree_pin_cap) {
+            if (w.h_tree_pin) ADB_HIP(hipHostFree(w.h_tree_pin));
+            w.h_tree_pin = nullptr;
+            w.h_tree_pin_cap = nt + nt / 2;
+            ADB_HIP(hipHostMalloc((void**)&w.h_tree_pin, w.h_tree_pin_cap * sizeof(int), hipHostMallocDefault));
+        }
+        std::memcpy(w.h_tree_pin, w.h_tree.data(), nt * sizeof(int));
+        w.tree_pack.reserve(nt);
+        ADB_HIP(hipMemcpyAsync(w.tree_pack.p, w.h_tree_pin, nt * sizeof(int), hipMemcpyHostToDevice, w.stream));
+    }
     ADB_HIP(hipEventRecord(w.ev_grp, w.stream));
     // the host vectors stay alive (members of w) until the copies have run
     w.Ginv.reserve((size_t)w.h_grp_moff.back());
@@ -1144,7 +1245,13 @@ void assemble_system(World& w) {
         ProfScope ps(w, PK_BLOCK_CHOL, 0.0);
         if (w.prof.on) {
             double fl = 0.0;
-            for (int g = 0; g < w.n_groups; g++) fl += group_inv_flops(w.h_grp_off[g + 1] - w.h_grp_off[g]);
+            for (int g = 0; g < w.n_groups; g++)
+                if (w.h_grp_off[g + 1] - w.h_grp_off[g] <= GMAX) fl += group_inv_flops(w.h_grp_off[g + 1] - w.h_grp_off[g]);
+            // the trees: block products, substitutions, factors and their inverses
+            for (int tr = 0; tr < w.n_trees; tr++) {
+                const int* T = w.h_tree.data() + w.n_trees + w.hg_tree_tab[tr];
+                fl += 3456.0 * (T[2] + T[3]) + 1728.0 * T[2] + 1152.0 * T[0];
+            }
             ps.flops = fl;
         }
         static_assert(GMAX == 8, "size classes 5..8 and 1..4");
@@ -1154,6 +1261,7 @@ void assemble_system(World& w) {
             hipLaunchKernelGGL(k_group_inv, dim3(nb), dim3(256), 0, w.stream, w.glist, w.n_glist[0], n4, w.grp_off,
                                w.grp_body, w.grp_moff, w.row_ptr.p, w.col_idx.p, w.Hval.p, w.Ginv.p);
         ADB_HIP(hipGetLastError());
+        tree_factor(w);
     }
 }
 

@@ -27,6 +27,7 @@
 // flag of the previous batch while the current one runs.
 #include <cmath>
 #include <functional>
+#include <type_traits>
 #include "dmath.h"
 #include "world.h"
 
@@ -136,7 +137,10 @@ __device__ double wg_sum(double v, double* sh) {
 // Preconditioner of the body groups: z = M_g^-1 r on group g's rows (n = 12
 // bodies <= GN); group tables hold B entries, those past *count are unused.
 constexpr int GN = 96;
-struct Groups { const int* off; const int* body; const long long* moff; const double* Minv; const int* count; };
+struct Groups {
+    const int* off; const int* body; const long long* moff; const double* Minv; const int* count;
+    const int* tree; const int* tab;      // trees: the group's table (tree.h) at tab + tree[g]; -1: an explicit inverse
+};
 
 // Batched worlds: each scene's residual test, |r_s|^2 <= rtol^2 |b_s|^2, from
 // the groups' r.r (groups are numbered scene by scene); first = those of
@@ -288,12 +292,13 @@ __global__ __launch_bounds__(64 * SP_ROWS, U == 8 && !SPLIT ? 3 : 4) void k_pcg_
 // scalars and partials; body and the lane's part of the inverse (48 values in
 // flight); the vectors.
 constexpr int UPD_T = 2 * GN, GH = GN / 2;
-struct GroupRow { double M[GH]; size_t k; int m, j0; bool on; };      // k: the row's element; columns [j0, j0 + 6 m)
-__device__ __forceinline__ void load_group(GroupRow& q, const Groups& G, int gi, int t) {
+struct GroupRow { double M[GH]; size_t k; int m, j0, tree; bool on; };      // k: the row's element; columns [j0, j0 + 6 m)
+template <bool TREES> __device__ __forceinline__ void load_group(GroupRow& q, const Groups& G, int gi, int t) {
     const int cnt = *G.count, o0 = G.off[gi], o1 = G.off[gi + 1];
     const double* M = G.Minv + G.moff[gi];
     const int i = t % GN, h = t / GN;
-    q.m = gi < cnt ? o1 - o0 : 0;
+    q.tree = TREES && gi < cnt ? G.tree[gi] : -1;
+    q.m = gi < cnt && q.tree < 0 ? o1 - o0 : 0;
     q.on = i < 12 * q.m;
     q.j0 = h * 6 * q.m;
     q.k = 0;
@@ -307,13 +312,16 @@ __device__ __forceinline__ void load_group(GroupRow& q, const Groups& G, int gi,
             for (int u = 6 * s; u < 6 * s + 6; u++) q.M[u] = M[u * 12 * q.m];
         }
 }
-template <bool FIRST, int U, bool SPLIT>
+// TREES: some group may be a tree component (tree.h; a world has such groups
+// or not, and their code and LDS would cost the others 3 us a launch).
+template <bool FIRST, int U, bool SPLIT, bool TREES>
 __global__ __launch_bounds__(UPD_T) void k_pcg_update(int kloc, int nbS, Groups G,
                                                       double* __restrict__ p, const double* __restrict__ y,
                                                       double* __restrict__ x, double* __restrict__ r, double* __restrict__ z,
                                                       const double* __restrict__ partA, double* __restrict__ partB,
                                                       double* __restrict__ grr, double* scal) {
-    __shared__ double rs[GN];
+    __shared__ double rs[TREES ? 12 * TREE_MAX : GN];
+    __shared__ int tab[TREES ? TREE_SOLVE_INTS : 1];
     __shared__ double half2[GN];
     __shared__ double red[UPD_T / 64][2], sh1[UPD_T / 64][1];
     const int t = threadIdx.x;
@@ -325,7 +333,7 @@ __global__ __launch_bounds__(UPD_T) void k_pcg_update(int kloc, int nbS, Groups 
     }
     const int ng = *G.count;
     GroupRow q;
-    load_group(q, G, blockIdx.x, t);
+    load_group<TREES>(q, G, blockIdx.x, t);
     const bool vec = t < GN;
     double xk = 0.0, pk = 0.0, yk = 0.0, rk = 0.0;
     if (q.on && vec) {
@@ -349,6 +357,30 @@ __global__ __launch_bounds__(UPD_T) void k_pcg_update(int kloc, int nbS, Groups 
     }
     double a0 = 0.0, a1 = 0.0;
     for (int gi = blockIdx.x; gi < ng;) {
+        double pz = 0.0, pr = 0.0;
+        if (TREES && q.tree >= 0) {
+            const int* T = G.tab + q.tree;
+            const int ti = tree_solve_ints(T[0], T[1], T[2]);
+            for (int i = t; i < ti; i += UPD_T) tab[i] = T[i];
+            __syncthreads();
+            const TreeTab tt = tree_tab(tab);
+            for (int i = t; i < 12 * tt.n; i += UPD_T) {
+                const size_t k = 12 * (size_t)tt.body[i / 12] + i % 12;
+                const double rn = FIRST ? -y[k] : r[k] - alpha * y[k];
+                x[k] = FIRST ? 0.0 : x[k] + alpha * p[k];
+                if (FIRST) p[k] = 0.0;
+                r[k] = rn;
+                rs[i] = rn;
+            }
+            __syncthreads();
+            tree_solve<UPD_T>(tt, G.Minv + G.moff[gi], rs);
+            for (int i = t; i < 12 * tt.n; i += UPD_T) {
+                const size_t k = 12 * (size_t)tt.body[i / 12] + i % 12;
+                const double rn = r[k], zn = rs[i];
+                z[k] = zn;
+                pz += rn * zn; pr += rn * rn;
+            }
+        }
         if (q.on && vec) {
             x[q.k] = FIRST ? 0.0 : xk + alpha * pk;
             rk = FIRST ? -yk : rk - alpha * yk;
@@ -369,7 +401,6 @@ __global__ __launch_bounds__(UPD_T) void k_pcg_update(int kloc, int nbS, Groups 
         }
         if (!vec && q.on) half2[i] = zi;
         __syncthreads();
-        double pz = 0.0, pr = 0.0;
         if (vec && q.on) {
             zi += half2[i];
             z[q.k] = zi;
@@ -378,7 +409,7 @@ __global__ __launch_bounds__(UPD_T) void k_pcg_update(int kloc, int nbS, Groups 
         // the next group's loads run under the sums
         const int gj = gi + gridDim.x;
         if (gj < ng) {
-            load_group(q, G, gj, t);
+            load_group<TREES>(q, G, gj, t);
             if (q.on && vec) {
                 yk = y[q.k];
                 if (!FIRST) { xk = x[q.k]; pk = p[q.k]; rk = r[q.k]; }
@@ -402,6 +433,7 @@ __global__ __launch_bounds__(UPD_T) void k_pcg_update(int kloc, int nbS, Groups 
 static Groups groups_of(World& w) {
     Groups G;
     G.off = w.grp_off; G.body = w.grp_body; G.moff = w.grp_moff; G.Minv = w.Ginv.p; G.count = w.grp_n;
+    G.tree = w.grp_tree; G.tab = w.tree_pack.p + w.n_trees;
     return G;
 }
 
@@ -428,9 +460,14 @@ template <bool FIRST> static void launch_update(World& w, int k, double* p, cons
         hipLaunchKernelGGL(kernel, dim3(nbU), dim3(UPD_T), 0, w.stream, k, nbS, groups_of(w), p, y, w.pcg_xo, w.pcg_r.p, w.pcg_z.p,
                            partA, partB, w.S > 1 ? partB + 2 * nbU : (double*)nullptr, w.scal.p);
     };
-    if (FIRST || nbS <= 64) go(k_pcg_update<FIRST, 1, false>);
-    else if (nbS <= 512) go(k_pcg_update<FIRST, 8, false>);
-    else go(k_pcg_update<FIRST, 8, true>);
+    auto form = [&](auto trees) {
+        constexpr bool T = decltype(trees)::value;
+        if (FIRST || nbS <= 64) go(k_pcg_update<FIRST, 1, false, T>);
+        else if (nbS <= 512) go(k_pcg_update<FIRST, 8, false, T>);
+        else go(k_pcg_update<FIRST, 8, true, T>);
+    };
+    if (w.n_trees > 0) form(std::true_type{});
+    else form(std::false_type{});
 }
 static void launch_scene_stop(World& w, int first) {
     const double* grr = w.partial.p + spmv_wgs(w.B) + 2 * update_wgs(w.B);
@@ -485,7 +522,7 @@ int pcg_solve(World& w, double* dq_out, int* iters, const std::function<void()>&
     if (use_graph) {
         const void* key[] = {w.row_ptr.p, w.col_idx.p, w.Hval.p, w.Ginv.p, w.pcg_xo, w.pcg_r.p, w.pcg_z.p, w.pcg_p.p,
                              w.pcg_p2.p, w.pcg_Ap.p, w.partial.p, w.scal.p, w.grp_off, w.grp_body, w.grp_moff,
-                             w.grp_n, w.sc_goff.p, w.pcg_sbb.p};
+                             w.grp_n, w.sc_goff.p, w.pcg_sbb.p, w.n_trees ? w.tree_pack.p + w.n_trees : nullptr};
         static_assert(sizeof key / sizeof key[0] == World::PCG_GRAPH_KEYS, "graph key size");
         const int BATCH = w.tune.pcg_batch;
         bool same = w.pcg_graph != nullptr && w.pcg_graph_batch == BATCH;

@@ -7,6 +7,7 @@
 #include <string>
 #include <vector>
 #include "../../include/adb_capi.h"
+#include "tree.h"
 
 namespace adb {
 
@@ -205,6 +206,14 @@ struct World {
     hipEvent_t ev_grp = nullptr;     // the last upload from the staging buffer
     long long* grp_moff = nullptr;
     int *grp_off = nullptr, *grp_body = nullptr, *glist = nullptr, *grp_n = nullptr;
+    int* grp_tree = nullptr;         // per group: its table's offset in the tree tables, or -1
+    DBuf<int> tree_pack;             // tree groups' ids (n_trees), then their tables (tree.h)
+    int n_trees = 0;
+    int* h_tree_pin = nullptr;
+    size_t h_tree_pin_cap = 0;
+    TreePlan tree_plan;
+    std::vector<int> h_tree, hg_tree, hg_tree_tab, hg_tree_ne, hg_cpar, hg_ccnt, hg_cid, hg_loc, hg_boff, hg_bods, hg_poff, hg_prs,
+        hg_fill, hg_tabs;
     DBuf<double> Ginv;
     int n_groups = 0;
     std::vector<int> h_glist;
@@ -226,7 +235,7 @@ struct World {
     hipEvent_t ev_phase[2] = {nullptr, nullptr};   // contact terms + assembly on the stream: start, end
     bool use_graphs = true;          // ADB_PCG_GRAPH=0 turns graph capture off
     hipGraphExec_t pcg_graph = nullptr;   // one captured PCG batch
-    static constexpr int PCG_GRAPH_KEYS = 18;
+    static constexpr int PCG_GRAPH_KEYS = 19;
     const void* pcg_graph_key[PCG_GRAPH_KEYS] = {};   // buffer addresses the graph was captured with
     double* h_scal = nullptr;        // pinned host copies of the PCG scalars (2 x 8)
     hipEvent_t pcg_ev[2] = {nullptr, nullptr};
@@ -327,6 +336,7 @@ void hash_ccd(World& w, const double* X0, const double* X1, unsigned long long* 
 void contact_terms(World& w);                                                            // contact.hip
 void assemble_structure(World& w, bool forked);                                         // assemble.hip
 void assemble_system(World& w);                                                          // assemble.hip
+void tree_factor(World& w);                                                              // tree.hip
 // `after` (if given) queues work behind a short solve's stop test, before
 // its wait; *after_valid tells whether that solve was then complete (else
 // the work ran on an unfinished x and must be queued again)

@@ -587,7 +587,10 @@ static void free_world(World& w) {
     if (w.pcg_graph) (void)hipGraphExecDestroy(w.pcg_graph);
     w.pcg_graph = nullptr;
     w.grp_pack.free_();
-    w.grp_moff = nullptr; w.grp_off = w.grp_body = w.glist = w.grp_n = nullptr;
+    w.grp_moff = nullptr; w.grp_off = w.grp_body = w.glist = w.grp_n = w.grp_tree = nullptr;
+    w.tree_pack.free_();
+    if (w.h_tree_pin) (void)hipHostFree(w.h_tree_pin);
+    w.h_tree_pin = nullptr; w.h_tree_pin_cap = 0;
     if (w.h_grp_pack) (void)hipHostFree(w.h_grp_pack);
     w.h_grp_pack = nullptr; w.h_grp_pack_cap = 0;
     if (w.ev_grp) (void)hipEventDestroy(w.ev_grp);

@@ -58,3 +58,59 @@ def test_direction_of_independent_stacks(B, batched):
         tol = 1e-7 * np.abs(do).max()
         np.testing.assert_allclose(dq[STACK * s:STACK * (s + 1)], do, rtol=0, atol=tol)
     np.testing.assert_allclose(dq[n_stack * STACK:], np.repeat(ds.reshape(1, 12), B - n_stack * STACK, axis=0), rtol=0, atol=tol)
+
+
+def column(n, rng):
+    gap = 0.5 * np.sqrt(D_HAT)
+    return [(rng.uniform(-0.05, 0.05), (1.0 + gap) * i, rng.uniform(-0.05, 0.05)) for i in range(n)], []
+
+
+def wall(w, h, d):
+    def make(rng):
+        step = 1.0 + 0.5 * np.sqrt(D_HAT)
+        return [(step * i, step * j, step * k) for k in range(d) for j in range(h) for i in range(w)], []
+    return make
+
+
+def shelf(n, rng):
+    # columns of 10 cubes, each on a static cube of its own
+    gap = 0.5 * np.sqrt(D_HAT)
+    pos = [(3.0 * c, (1.0 + gap) * i, 0.0) for c in range(n) for i in range(11)]
+    return pos, [11 * c for c in range(n)]
+
+
+SHAPES = {
+    # a path one body longer than an explicit inverse takes; the shortest and
+    # the longest that a component's factors take, and one more or less (which
+    # keep the small groups)
+    "path9": lambda rng: column(9, rng), "path16": lambda rng: column(16, rng), "path17": lambda rng: column(17, rng), "path256": lambda rng: column(256, rng), "path257": lambda rng: column(257, rng),
+    # cycles and fill: every cube of a wall touches its eight neighbours
+    "wall3x4": wall(3, 4, 1), "wall4x10": wall(4, 10, 1),
+    # too dense to eliminate: 26 neighbours
+    "block4x4x4": wall(4, 4, 4),
+    "static": lambda rng: shelf(3, rng),
+}
+
+
+@pytest.mark.parametrize("psd", [1, 0])
+@pytest.mark.parametrize("shape", list(SHAPES))
+def test_direction_of_one_component(shape, psd):
+    """Contact components as one preconditioner group (more than 8 bodies):
+    the direction against the oracle's direct solve; tolerance as above."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    v, f, e = scenes.cube_mesh()
+    rng = np.random.default_rng(7)
+    pos, static = SHAPES[shape](rng)
+    mass = rng.uniform(500.0, 2000.0, len(pos))
+    mass[static] = -1.0
+    bodies = [dict(verts=v, tris=f, edges=e, R=np.eye(3), p=q, mass=float(m)) for q, m in zip(pos, mass)]
+    sc = scenes.build_scene(bodies)
+    p = default_params(d_hat=D_HAT, mu=0.4, enable_ground=0, psd=psd)
+    w, ow = World(sc, p), O.OracleWorld(sc, p)
+    pt, ee, _ = ow.collision_set()
+    assert len(pt) + len(ee) > 10 * len(pos)
+    rg, dg = w.newton_direction()
+    ro, do = ow.newton_direction()
+    assert rg == ro == 0
+    np.testing.assert_allclose(dg, do, rtol=0, atol=1e-7 * np.abs(do).max())
