@@ -205,9 +205,10 @@ __global__ void k_chunk_owner(int npb, const int* __restrict__ npd, const int* _
 
 // ---- the block-row structure, vertex-ground starts, chunk table and the
 // host's copy of the pair lists in one workgroup (the launches of the kernels
-// above, which stay for large B + pair counts, each cost more than their work
-// in the light phase of a scene)
-constexpr int STRUCT_T = 1024, STRUCT_MAX = 1 << 16;
+// above cost more than their work there).  For worlds whose body lists fit its
+// LDS; beyond, one workgroup takes several passes over them in global memory
+// (27 000 bodies 282 us, against 50 us for the kernels above).
+constexpr int STRUCT_T = 1024;
 // exclusive scan of in[0, n) into out[0, n], out[n] = the total, by one
 // workgroup of STRUCT_T threads (contiguous ranges per thread); returns the total
 __device__ int block_scan_excl(const int* in, int* out, int n, int* sh) {
@@ -254,7 +255,7 @@ struct StructArgs {
     int* vg_start; int* chunk_n; int* chunk_off; int* chunk_pair; int* counts;
     int* host_pack;   // [pair count, npb pair_lo, npb pair_hi, npb + 1 pair_start]
 };
-// body arrays of at most STRUCT_LB entries (B + 1) and chunk arrays of at most
+// body arrays (B + 1 <= STRUCT_LB entries) and chunk arrays of at most
 // 5 STRUCT_LB / 2 entries (np + 1) are staged in LDS (40 KB, reused): the
 // phases between barriers then read their inputs from LDS instead of global
 // memory, and the outputs are written once
@@ -263,12 +264,11 @@ __global__ __launch_bounds__(STRUCT_T) void k_structure(StructArgs a) {
     __shared__ int sh[STRUCT_T / 64];
     __shared__ int lb[5 * STRUCT_LB];
     const int np = pair_count(a.npb, a.npd), t = threadIdx.x, B = a.B;
-    const bool lb_on = B + 1 <= STRUCT_LB;
-    int* up = lb_on ? lb : a.up_start;
-    int* low = lb_on ? lb + STRUCT_LB : a.low_start;
-    int* vgs = lb_on ? lb + 2 * STRUCT_LB : a.vg_start;
-    int* rc = lb_on ? lb + 3 * STRUCT_LB : a.rowcnt;
-    int* rp = lb_on ? lb + 4 * STRUCT_LB : a.row_ptr;
+    int* up = lb;
+    int* low = lb + STRUCT_LB;
+    int* vgs = lb + 2 * STRUCT_LB;
+    int* rc = lb + 3 * STRUCT_LB;
+    int* rp = lb + 4 * STRUCT_LB;
     // k_body_ranges and k_vg_start without their binary searches (chains of
     // dependent loads): each body's first entry in a list sorted by body is
     // marked, the other bodies get the list length, and a suffix minimum over
@@ -292,10 +292,9 @@ __global__ __launch_bounds__(STRUCT_T) void k_structure(StructArgs a) {
     for (int b = t; b < B; b += STRUCT_T) rc[b] = (low[b + 1] - low[b]) + 1 + (up[b + 1] - up[b]);
     __syncthreads();
     block_scan_excl(rc, rp, B, sh);
-    if (lb_on)
-        for (int b = t; b <= B; b += STRUCT_T) {
-            a.up_start[b] = up[b]; a.low_start[b] = low[b]; a.vg_start[b] = vgs[b]; a.row_ptr[b] = rp[b];
-        }
+    for (int b = t; b <= B; b += STRUCT_T) {
+        a.up_start[b] = up[b]; a.low_start[b] = low[b]; a.vg_start[b] = vgs[b]; a.row_ptr[b] = rp[b];
+    }
     // k_fill_cols
     for (int b = t; b < B; b += STRUCT_T) {
         int k = rp[b];
@@ -318,8 +317,13 @@ __global__ __launch_bounds__(STRUCT_T) void k_structure(StructArgs a) {
     for (int p = t; p < np; p += STRUCT_T) cn[p] = (a.pair_start[p + 1] - a.pair_start[p] + PCH - 1) / PCH;
     __syncthreads();
     const int nch = block_scan_excl(cn, co, np, sh);
-    for (int p = t; p < np; p += STRUCT_T)
-        for (int c = co[p]; c < co[p + 1]; c++) a.chunk_pair[c] = p;
+    // each chunk looks its pair up: few pairs may own most of the chunks (386
+    // pairs of 1500 crowded bodies, a thread a pair: the kernel 160 -> 38 us)
+    for (int c = t; c < nch; c += STRUCT_T) {
+        int lo = 0, hi = np;
+        while (hi - lo > 1) { const int mid = (lo + hi) / 2; if (co[mid] <= c) lo = mid; else hi = mid; }
+        a.chunk_pair[c] = lo;
+    }
     if (lc_on)
         for (int p = t; p <= np; p += STRUCT_T) a.chunk_off[p] = co[p];
     if (t == 0) a.counts[3] = nch;
@@ -1151,7 +1155,7 @@ void assemble_structure(World& w, bool forked) {
     const int max_chunks = (np + nc / PCH + 7) / 8 * 8;
     w.chunk_blk.reserve(std::max(max_chunks, 1));
     w.chunk_part.reserve(PART * (size_t)std::max(max_chunks, 1));
-    const bool one_wg = B + np <= STRUCT_MAX && !w.general_paths;
+    const bool one_wg = B + 1 <= STRUCT_LB && !w.general_paths;
     if (one_wg) {
         // 3. block rows, vertex-ground starts and chunks in one workgroup
         w.pair_pack.reserve(3 * (size_t)np + 2);
