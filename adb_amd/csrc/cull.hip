@@ -355,6 +355,10 @@ __global__ void k_sweep_pairs(int B, const unsigned long long* __restrict__ keys
 //      segment, from which the line search's trial sets are filtered.
 // Boxes only cull; the FP64 predicate decides, so the sets equal those of the
 // all-pairs tests (model/thread_local_culling.cpp:209-386 pt/ee_col_set_task).
+// fewest edges of a slice of the EE pass: each slice stages the other body's
+// edges again, which for small meshes costs more than the tests it splits
+// (cards of 18 edges, 9900 pairs: 515 us in 4 slices, 410 us in one)
+constexpr int EE_SLICE = 96;
 constexpr int PAIRS_PT = 4;                    // box tests per thread per round
 // workgroups per body pair: 2 PT passes + the EE pass in ee_slices slices (tuning)
 constexpr int QCAP = NB_THREADS * PAIRS_PT * 3 / 2; // candidate queue (i << 16 | j: staged indices < 2^16)
@@ -607,7 +611,9 @@ __global__ __launch_bounds__(NB_THREADS) void k_pair_narrow(NarrowArgs a) {
             int endA = offA[bA + 1];
             if (pass == 2) {
                 const int len = endA - curA, q = task - 2;
-                const int s0 = curA + (int)((long long)len * q / a.ee_slices), s1 = curA + (int)((long long)len * (q + 1) / a.ee_slices);
+                const int ns = min(a.ee_slices, (len + EE_SLICE - 1) / EE_SLICE);
+                if (q >= ns) continue;
+                const int s0 = curA + (int)((long long)len * q / ns), s1 = curA + (int)((long long)len * (q + 1) / ns);
                 curA = s0; endA = s1;
             }
             while (curA < endA) {
