@@ -3,7 +3,9 @@
 // pt_collision_time / ee_collision_time (model/collision.cpp:299-348, exposed by
 // python/bindings.cpp:81-82) and the distance type + squared distance pair
 // (model/geometry.cpp:101-112, model/abd.cpp:353-354), one entry per lane.
+#include <cstring>
 #include <mutex>
+#include "staging.h"
 #include "dmath.h"
 #include "world.h"
 
@@ -59,15 +61,11 @@ extern "C" int adb_ee_distance_batched(int n, const double* x, int* type, double
 }
 
 static double single_toi(int is_ee, const double x[24]) {
-    double *dx = nullptr, *dt = nullptr;
-    double out = -1.0;
-    if (hipMalloc((void**)&dx, 24 * sizeof(double)) == hipSuccess && hipMalloc((void**)&dt, sizeof(double)) == hipSuccess) {
-        hipMemcpy(dx, x, 24 * sizeof(double), hipMemcpyHostToDevice);
-        int rc = is_ee ? adb_ee_collision_time_batched(1, dx, dt, nullptr) : adb_pt_collision_time_batched(1, dx, dt, nullptr);
-        if (rc == ADB_OK && hipDeviceSynchronize() == hipSuccess) hipMemcpy(&out, dt, sizeof(double), hipMemcpyDeviceToHost);
-    }
-    hipFree(dx); hipFree(dt);
-    return out;
+    double* m = host_staging().get();
+    if (!m) return -1.0;
+    std::memcpy(m, x, 24 * sizeof(double));
+    const int rc = is_ee ? adb_ee_collision_time_batched(1, m, m + 24, nullptr) : adb_pt_collision_time_batched(1, m, m + 24, nullptr);
+    return rc == ADB_OK && hipStreamSynchronize(nullptr) == hipSuccess ? m[24] : -1.0;
 }
 extern "C" double adb_pt_collision_time(const double x[24]) { return single_toi(0, x); }
 extern "C" double adb_ee_collision_time(const double x[24]) { return single_toi(1, x); }

@@ -39,7 +39,9 @@
 // 22 us a call, 2e5 EE contacts (a tenth mollified) 4458 -> 200 us.
 #include <cstdio>
 #include <algorithm>
+#include <cstring>
 #include "dmath.h"
+#include "staging.h"
 #include "terms.h"
 #include "world.h"
 
@@ -1349,30 +1351,24 @@ extern "C" int adb_ipc_hess_ee_12x12_batched(const adb_kernel_config* cfg, int n
 
 template <int IS_EE>
 static int single_hess(const adb_kernel_config* cfg, const double x[12], int type, double dist, double H[144], double g[12], double* moll) {
-    double *dx = nullptr, *dd = nullptr, *dH = nullptr, *dg = nullptr, *dm = nullptr;
-    int* dt = nullptr;
-    int rc = ADB_OK;
-    if (hipMalloc((void**)&dx, 12 * sizeof(double)) != hipSuccess || hipMalloc((void**)&dd, sizeof(double)) != hipSuccess ||
-        hipMalloc((void**)&dH, 144 * sizeof(double)) != hipSuccess || hipMalloc((void**)&dg, 12 * sizeof(double)) != hipSuccess ||
-        hipMalloc((void**)&dm, sizeof(double)) != hipSuccess || hipMalloc((void**)&dt, sizeof(int)) != hipSuccess) {
-        rc = ADB_E_HIP;
-    } else {
-        if (hipMemcpy(dx, x, 12 * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(dd, &dist, sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(dt, &type, sizeof(int), hipMemcpyHostToDevice) != hipSuccess) rc = ADB_E_HIP;
-        if (rc == ADB_OK) {
-            if (IS_EE) rc = adb_ipc_hess_ee_12x12_batched(cfg, 1, dx, dt, dd, dH, dg, dm, nullptr);
-            else rc = adb_ipc_hess_pt_12x12_batched(cfg, 1, dx, dt, dd, dH, dg, nullptr);
-        }
-        if (rc == ADB_OK && hipDeviceSynchronize() != hipSuccess) rc = ADB_E_HIP;
-        if (rc == ADB_OK) {
-            if (hipMemcpy(H, dH, 144 * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess ||
-                hipMemcpy(g, dg, 12 * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess) rc = ADB_E_HIP;
-            if (IS_EE && moll && hipMemcpy(moll, dm, sizeof(double), hipMemcpyDeviceToHost) != hipSuccess) rc = ADB_E_HIP;
-        }
-    }
-    (void)hipFree(dx); (void)hipFree(dd); (void)hipFree(dH); (void)hipFree(dg); (void)hipFree(dm); (void)hipFree(dt);
-    return rc;
+    double* m = host_staging().get();
+    if (!m) return ADB_E_HIP;
+    // x (12), dist, type | H (144), g (12), moll
+    double *mH = m + 16, *mg = mH + 144, *mm = mg + 12;
+    static_assert(16 + 144 + 12 + 1 <= HostStaging::N, "single contact in the staging page");
+    std::memcpy(m, x, 12 * sizeof(double));
+    m[12] = dist;
+    int* mt = reinterpret_cast<int*>(m + 13);
+    *mt = type;
+    int rc;
+    if (IS_EE) rc = adb_ipc_hess_ee_12x12_batched(cfg, 1, m, mt, m + 12, mH, mg, mm, nullptr);
+    else rc = adb_ipc_hess_pt_12x12_batched(cfg, 1, m, mt, m + 12, mH, mg, nullptr);
+    if (rc == ADB_OK && hipStreamSynchronize(nullptr) != hipSuccess) rc = ADB_E_HIP;
+    if (rc != ADB_OK) return rc;
+    std::memcpy(H, mH, 144 * sizeof(double));
+    std::memcpy(g, mg, 12 * sizeof(double));
+    if (IS_EE && moll) *moll = *mm;
+    return ADB_OK;
 }
 extern "C" int adb_ipc_hess_pt_12x12(const adb_kernel_config* cfg, const double pt[12], int type, double dist, double H[144], double g[12]) {
     return single_hess<0>(cfg, pt, type, dist, H, g, nullptr);
