@@ -194,13 +194,13 @@ __global__ void k_pair_chunks(int npb, const int* __restrict__ npd, const int* _
     nch[p] = p < np ? (pair_start[p + 1] - pair_start[p] + PCH - 1) / PCH : 0;
 }
 // chunk_off = exclusive scan of nch (npb + 1 entries); the chunk count also
-// goes to counts[3] for the byte accounting
+// goes to counts[4] for the byte accounting
 __global__ void k_chunk_owner(int npb, const int* __restrict__ npd, const int* __restrict__ chunk_off, int* __restrict__ chunk_pair,
                               int* __restrict__ counts) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     const int np = pair_count(npb, npd);
     if (k < np) for (int c = chunk_off[k]; c < chunk_off[k + 1]; c++) chunk_pair[c] = k;
-    if (k == 0) counts[3] = chunk_off[np];
+    if (k == 0) counts[4] = chunk_off[np];
 }
 
 // ---- the block-row structure, vertex-ground starts, chunk table and the
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(STRUCT_T) void k_structure(StructArgs a) {
     }
     if (lc_on)
         for (int p = t; p <= np; p += STRUCT_T) a.chunk_off[p] = co[p];
-    if (t == 0) a.counts[3] = nch;
+    if (t == 0) a.counts[4] = nch;
     // the pair lists for the host's group building, one copy
     if (t == 0) a.host_pack[0] = np;
     for (int p = t; p < np; p += STRUCT_T) { a.host_pack[1 + p] = a.pair_lo[p]; a.host_pack[1 + a.npb + p] = a.pair_hi[p]; }
@@ -1237,7 +1237,7 @@ void assemble_system(World& w) {
         // every contact record read once (D = 3: 75 doubles, 6: 102, 9: 147), its id,
         // pair side and class; one partial (3 blocks + 2 gradients) written per chunk
         ProfScope ps(w, PK_ASM_REDUCE, 24.0 * nc);
-        ps.counts(prof_snapshot(w, w.ccount.p), 600.0, 816.0, 1176.0, 8.0 * PART);
+        ps.counts(prof_snapshot(w, w.ccount.p), 600.0, 816.0, 1176.0, 1176.0, 8.0 * PART);
         hipLaunchKernelGGL(k_pair_reduce, dim3(max_chunks), dim3(256), 0, w.stream, a, w.chunk_blk.p, w.chunk_part.p);
         ADB_HIP(hipGetLastError());
     }

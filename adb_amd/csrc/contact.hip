@@ -11,12 +11,14 @@
 // translation-free space of the n + 1 points it involves, and appends it to
 // that class's list; then one thread per contact:
 //   class 1 (two points, D = 3): closed-form projection (k_contact_small<1>);
-//   class 2 (three points, D = 6): record fields (k_contact_scalars2), then
-//     cyclic Jacobi on the packed 6 x 6 matrix in registers (k_contact_pk2);
-//   class 3 (four points, or any mollified EE, D = 9): the 9 x 9 matrix into
-//     the record, then cyclic Jacobi in registers (k_contact_c3r, nine
-//     threads per contact building the matrix and a tenth the other record
-//     fields, then k_contact_psd9, one thread per contact, on a side stream).
+//   class 2 (three points, D = 6): record fields (k_contact_scalars2) and the
+//     projection, 3 x 3 in the contact's frame (k_contact_pk2, side stream);
+//   class 3 (point-plane, edge-edge interior, D = 9): the whole record, 5 x 5
+//     in the contact's frame (k_contact_plane, side stream);
+//   class 4 (mollified edge pairs, D = 9): the 9 x 9 matrix into the record,
+//     then cyclic Jacobi in registers (k_contact_c3r, nine threads per contact
+//     building the matrix and a tenth the other record fields, then
+//     k_contact_psd9, one thread per contact, on a side stream).
 // Each contact writes a compact body-space record (world.h) that the
 // assembly expands into its four 12 x 12 blocks; the class 1 and class 2
 // record kernels stage it per wavefront in LDS and store it cooperatively
@@ -448,8 +450,8 @@ __device__ __forceinline__ bool contact_ids(const WorldArgs& a, int cid, int& id
 }
 
 // Class of an active contact by the points its barrier depends on:
-// 1 = two points (D = 3), 2 = three points (D = 6), 3 = four points (D = 9,
-// also every mollified edge-edge contact).  Inactive contacts (d >= d_hat)
+// 1 = two points (D = 3), 2 = three points (D = 6), 3 = four points (D = 9),
+// 4 = every mollified edge-edge contact (D = 9).  Inactive contacts (d >= d_hat)
 // get an empty record here.
 __device__ __forceinline__ int classify_one(const WorldArgs& a, int cid) {
     int id0, id1, id2, id3;
@@ -464,11 +466,11 @@ __device__ __forceinline__ int classify_one(const WorldArgs& a, int cid) {
     if (d < a.kp.d_hat) {
         const int kind = is_ee ? ee_map(type).kind : pt_map(type).kind;
         cls = kind == K_PP ? 1 : (kind == K_PL ? 2 : 3);
-        if (is_ee && cls < 3) {
+        if (is_ee) {
             // mollifier active: x = |(p1 - p0) x (p3 - p2)|^2 < eps_x |p0 - p1|^2 |p2 - p3|^2
             const double eps = a.kp.eps_x * sqn(p0 - p1) * sqn(p2 - p3);
             const d3 c = cross(p1 - p0, p3 - p2);
-            if (dot(c, c) < eps) cls = 3;
+            if (dot(c, c) < eps) cls = 4;
         }
     } else {
         a.rec[REC * (size_t)cid + R_D] = 0.0;
@@ -476,12 +478,13 @@ __device__ __forceinline__ int classify_one(const WorldArgs& a, int cid) {
         for (int i = 0; i < TKN; i++) tk[i] = 0.0;
         a.lam[cid] = 0.0;
     }
-    a.ccls[cid] = cls;
+    a.ccls[cid] = min(cls, 3);      // Helmert rows of the record
     return cls;
 }
 
 // Classification and the per-class lists (class 1 from the front of `list`,
-// class 2 from its back, class 3 in `list3`).  Device-scope atomics on one
+// class 2 from its back, class 3 from the front of `list3`, class 4 from its
+// back).  Device-scope atomics on one
 // address serialize (~11 ns each on gfx950), so the slots are claimed per
 // workgroup: each workgroup classifies a tile of rpt x CL_THREADS contacts,
 // counts its classes with LDS atomics (one per wavefront and class), takes
@@ -489,10 +492,10 @@ __device__ __forceinline__ int classify_one(const WorldArgs& a, int cid) {
 constexpr int CL_THREADS = 1024;
 constexpr int CL_RPT_MAX = 8;
 __global__ __launch_bounds__(CL_THREADS) void k_contact_classify(WorldArgs a, int rpt) {
-    __shared__ int lcnt[3], lbase[3];
+    __shared__ int lcnt[4], lbase[4];
     const int total = a.n_pt + a.n_ee;
     const int lane = __lane_id();
-    if (threadIdx.x < 3) lcnt[threadIdx.x] = 0;
+    if (threadIdx.x < 4) lcnt[threadIdx.x] = 0;
     __syncthreads();
     int cls_r[CL_RPT_MAX], pos_r[CL_RPT_MAX];
     const int base = blockIdx.x * CL_THREADS * rpt;
@@ -504,7 +507,7 @@ __global__ __launch_bounds__(CL_THREADS) void k_contact_classify(WorldArgs a, in
             const int cls = cid < total ? classify_one(a, cid) : 0;
             cls_r[r] = cls;
 #pragma unroll
-            for (int k = 1; k <= 3; k++) {
+            for (int k = 1; k <= 4; k++) {
                 const unsigned long long m = __ballot(cls == k);
                 if (m == 0ull) continue;
                 const int leader = __ffsll((long long)m) - 1;
@@ -516,7 +519,7 @@ __global__ __launch_bounds__(CL_THREADS) void k_contact_classify(WorldArgs a, in
         }
     }
     __syncthreads();
-    if (threadIdx.x < 3) lbase[threadIdx.x] = lcnt[threadIdx.x] ? atomicAdd(&a.counts[threadIdx.x], lcnt[threadIdx.x]) : 0;
+    if (threadIdx.x < 4) lbase[threadIdx.x] = lcnt[threadIdx.x] ? atomicAdd(&a.counts[threadIdx.x], lcnt[threadIdx.x]) : 0;
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < CL_RPT_MAX; r++) {
@@ -526,6 +529,7 @@ __global__ __launch_bounds__(CL_THREADS) void k_contact_classify(WorldArgs a, in
         if (cls == 1) a.list[lbase[0] + pos_r[r]] = cid;
         else if (cls == 2) a.list[total - 1 - (lbase[1] + pos_r[r])] = cid;
         else if (cls == 3) a.list3[lbase[2] + pos_r[r]] = cid;
+        else if (cls == 4) a.list3[total - 1 - (lbase[3] + pos_r[r])] = cid;
     }
 }
 
@@ -748,8 +752,7 @@ __device__ __forceinline__ void contact_small(const WorldArgs& a, const Stage& s
     grad_fields(nside0, w, gv, [&](int k, double v) { S[k - R_GRAD][l] = v; });
     stage_flush<24>(st, a.rec, REC, R_GRAD);
 }
-// Class 3 contacts (four points: point-plane, edge-edge interior, every
-// mollified edge-edge) in two launches.
+// Class 4 contacts (mollified edge pairs) in two launches.
 // k_contact_c3r: ten threads per contact.  Thread role r < 9 builds the entries
 // of the 9x9 Helmert-coordinate matrix K = (C (x) I3) Mred (C^T (x) I3) +
 // mollifier terms (C = h4 S^T, Cm the same for y = p1 - p0, z = p3 - p2) of
@@ -965,10 +968,10 @@ __device__ __forceinline__ void psd9(const WorldArgs& a, int cid) {
 // registers of their own code (two wavefronts per SIMD) while the Jacobi
 // holds ~280 (one).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_contact_c3r(WorldArgs a) {
-    const int n3 = a.counts[2];
-    const long long n = (long long)C3_ROLES * n3;
+    const int n4 = a.counts[3], last = a.n_pt + a.n_ee - 1;
+    const long long n = (long long)C3_ROLES * n4;
     for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long long)gridDim.x * blockDim.x) {
-        const int cid = a.list3[t / C3_ROLES], role = (int)(t % C3_ROLES);
+        const int cid = a.list3[last - (int)(t / C3_ROLES)], role = (int)(t % C3_ROLES);
         C3Ctx x;
         c3_setup(a, cid, x);
         if (role < 9) c3_kbuild(x, role);
@@ -976,8 +979,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     }
 }
 __global__ __launch_bounds__(64) void k_contact_psd9(WorldArgs a) {
-    const int n3 = a.counts[2];
-    for (int p = blockIdx.x * 64 + threadIdx.x; p < n3; p += gridDim.x * 64) psd9(a, a.list3[p]);
+    const int n4 = a.counts[3], last = a.n_pt + a.n_ee - 1;
+    for (int p = blockIdx.x * 64 + threadIdx.x; p < n4; p += gridDim.x * 64) psd9(a, a.list3[last - p]);
 }
 
 // record fields other than PK of a 3-point contact: D, friction, gradient, Z
@@ -1044,26 +1047,12 @@ __device__ __forceinline__ void scalars_c2(const WorldArgs& a, const Stage& st, 
     stage_flush<16>(st, a.rec, REC, R_Z);
 }
 
-// PK = V diag(max(w, 0)) V^T into R[R_PK], row-major N x N
-template <int N>
-__device__ __forceinline__ void write_projection(const double (&A)[N * (N + 1) / 2], const double (&V)[N * N], double* R) {
-    double wv[N];
-#pragma unroll
-    for (int k = 0; k < N; k++) wv[k] = fmax(A[PK_<N>(k, k)], 0.0);
-#pragma unroll
-    for (int p = 0; p < N; p++)
-#pragma unroll
-        for (int q = p; q < N; q++) {
-            double s = 0.0;
-#pragma unroll
-            for (int k = 0; k < N; k++) s += V[N * p + k] * wv[k] * V[N * q + k];
-            R[R_PK + N * p + q] = s;
-            R[R_PK + N * q + p] = s;
-        }
-}
-
-// PK of a 3-point contact (point-line distance): K = (C (x) I3) Mred (C^T (x) I3),
-// 6x6 Jacobi in registers
+// PK of a 3-point contact (point-line distance) in the frame of terms.h: f2
+// decouples (eigenvalue 2 B1 |gamma|^2), so what is left is 3 x 3, in f1 and
+// the two Helmert components of the normal displacement over the slots
+// (m, a, b).  Against the 6 x 6 Jacobi on the matrix of the point differences
+// 276 -> 138 us (2000 crowded bodies, 1.05e6 contacts), 99 -> 40 us (2000 spheres,
+// 3.9e5).
 __device__ __forceinline__ void pk_c2(const WorldArgs& a, int cid) {
     int id0, id1, id2, id3;
     const int is_ee = contact_ids(a, cid, id0, id1, id2, id3);
@@ -1074,49 +1063,149 @@ __device__ __forceinline__ void pk_c2(const WorldArgs& a, int cid) {
     const RedMap mp = is_ee ? ee_map(type) : pt_map(type);
     const double B1 = barrier_d1(d, a.kp.d_hat, a.kp.kappa);
     const double B2 = barrier_d2(d, a.kp.d_hat, a.kp.kappa);
-    double* R = a.rec + REC * (size_t)cid;
-    const int ka = mp.plus[0], kb = mp.plus[1], km = mp.minus[0];
-    const d3 pm = pick(P0, P1, P2, P3, km);
-    RedDist rd;
-    rd.init(K_PL, pick(P0, P1, P2, P3, ka) - pm, pick(P0, P1, P2, P3, kb) - pm, mk(0, 0, 0));
-    double A[21];
+    Frame F;
+    contact_frame(is_ee, type, P0, P1, P2, P3, F);
+    double gh[2], mh[2];
     {
-        double M[6][6];
+        auto at = [](const double v[4], int k) { return k == 0 ? v[0] : (k == 1 ? v[1] : (k == 2 ? v[2] : v[3])); };
+        const int km = mp.minus[0], ka = mp.plus[0], kb = mp.plus[1];
+        const double g0 = at(F.gam, km), g1 = at(F.gam, ka), g2 = at(F.gam, kb);
+        const double m0 = at(F.m1, km), m1 = at(F.m1, ka), m2 = at(F.m1, kb);
+        gh[0] = HS2 * (g0 - g1); gh[1] = HS6 * ((g0 + g1) - 2.0 * g2);
+        mh[0] = HS2 * (m0 - m1); mh[1] = HS6 * ((m0 + m1) - 2.0 * m2);
+    }
+    double A[6], kt = 2.0 * B1 * F.gn * F.gn;
+    {
+        const double dd = F.delta * F.delta, As = 2.0 * B1 + 4.0 * B2 * dd, kc = -2.0 * B1 * F.delta * F.gn, kn = -2.0 * B1 * dd;
+        A[PK_<3>(0, 0)] = 0.0;
 #pragma unroll
-        for (int u = 0; u < 6; u++)
+        for (int i = 0; i < 2; i++) {
+            A[PK_<3>(0, 1 + i)] = kc * mh[i];
 #pragma unroll
-            for (int v = u; v < 6; v++) {
-                const int m = u / 3, i = u % 3, n = v / 3, j = v % 3;
-                M[u][v] = B1 * rd.hess(m, i, n, j) + B2 * cmp(rd.g[m], i) * cmp(rd.g[n], j);
-                M[v][u] = M[u][v];
-            }
-        const double C[2][2] = {{-2.0 * HS2, -HS2}, {0.0, -3.0 * HS6}};
-#pragma unroll
-        for (int aa = 0; aa < 2; aa++)
-#pragma unroll
-            for (int i = 0; i < 3; i++)
-#pragma unroll
-                for (int bb = 0; bb < 2; bb++)
-#pragma unroll
-                    for (int j = 0; j < 3; j++) {
-                        double s = 0.0;
-#pragma unroll
-                        for (int m = 0; m < 2; m++)
-#pragma unroll
-                            for (int n = 0; n < 2; n++) s += C[aa][m] * C[bb][n] * M[3 * m + i][3 * n + j];
-                        if (3 * aa + i <= 3 * bb + j) A[PK_<6>(3 * aa + i, 3 * bb + j)] = s;
-                    }
+            for (int j = i; j < 2; j++) A[PK_<3>(1 + i, 1 + j)] = As * gh[i] * gh[j] + kn * mh[i] * mh[j];
+        }
     }
     if (a.kp.psd) {
-        double V[36];
-        jacobi_packed<6>(A, V);
-        write_projection<6>(A, V, R);
-    } else {
-#pragma unroll
-        for (int p = 0; p < 6; p++)
-#pragma unroll
-            for (int q = 0; q < 6; q++) R[R_PK + 6 * p + q] = A[PK_<6>(p, q)];
+        double V[9];
+        jacobi_packed<3>(A, V);
+        project_packed<3>(A, V);
+        kt = fmax(kt, 0.0);
     }
+    double* R = a.rec + REC * (size_t)cid + R_PK;
+    const double ign = 1.0 / F.gn;
+    const double e[2] = {gh[0] * ign, gh[1] * ign};
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    const double ni = cmp(F.n, i), nj = cmp(F.n, j), fi = cmp(F.f1, i), fj = cmp(F.f1, j);
+                    const double tt = A[PK_<3>(0, 0)] * (fi * fj) + kt * (cmp(F.f2, i) * cmp(F.f2, j));
+                    R[6 * (3 * q + i) + 3 * b + j] = e[q] * e[b] * tt + (e[q] * A[PK_<3>(0, 1 + b)] * (fi * nj) + e[b] * A[PK_<3>(0, 1 + q)] * (ni * fj)) +
+                                                     A[PK_<3>(1 + q, 1 + b)] * (ni * nj);
+                }
+}
+
+// Class 3 contacts (point-plane, edge-edge interior), one thread each: the
+// whole record from the frame of terms.h, the projection a 5 x 5 Jacobi in
+// registers.  Bound by the scattered points and the 1.2 KB record.  Ten
+// threads per contact building the 9 x 9 matrix in memory and a second kernel
+// projecting it there took 751 + 147 us for all class 3 and 4 contacts of 2000
+// crowded bodies; this takes 342 us, and 149 + 130 us are left for the
+// mollified ones.
+__device__ __forceinline__ void contact_plane(const WorldArgs& a, const Stage& st, bool valid) {
+    const int cid = st.cid, l = st.lane;
+    double (*S)[SLD] = st.S;
+    int id0, id1, id2, id3;
+    const int is_ee = contact_ids(a, cid, id0, id1, id2, id3);
+    const d3 P0 = ld3(a.X + 3 * (size_t)id0), P1 = ld3(a.X + 3 * (size_t)id1);
+    const d3 P2 = ld3(a.X + 3 * (size_t)id2), P3 = ld3(a.X + 3 * (size_t)id3);
+    const int type = a.ctype[cid];
+    const double d = a.cdist[cid];
+    const int nside0 = is_ee ? 2 : 1;
+    const double B1 = barrier_d1(d, a.kp.d_hat, a.kp.kappa);
+    const double B2 = barrier_d2(d, a.kp.d_hat, a.kp.kappa);
+    Frame F;
+    contact_frame(is_ee, type, P0, P1, P2, P3, F);
+    double M[15];
+    frame_matrix(F, B1, B2, M);
+    if (a.kp.psd) {
+        double V[25];
+        jacobi_packed<5>(M, V);
+        project_packed<5>(M, V);
+    }
+    {
+        double g[3];
+        helmert(F.gam, g);
+        const double ign = 1.0 / F.gn;
+#pragma unroll
+        for (int q = 0; q < 3; q++) g[q] *= ign;
+        // rows (q, i) of the 9 x 9 matrix, two rows a section
+#pragma unroll
+        for (int r0 = 0; r0 < 10; r0 += 2) {
+#pragma unroll
+            for (int r = r0; r < r0 + 2 && r < 9; r++) {
+                const int q = r / 3, i = r % 3;
+                const double ni = cmp(F.n, i), f1 = cmp(F.f1, i), f2 = cmp(F.f2, i);
+                // the row's weights of f1, f2 and n at column component j, Helmert row b
+                const double u1 = M[PK_<5>(0, 0)] * f1 + M[PK_<5>(0, 1)] * f2, u2 = M[PK_<5>(0, 1)] * f1 + M[PK_<5>(1, 1)] * f2;
+                const double c1 = g[q] * u1 + M[PK_<5>(0, 2 + q)] * ni, c2 = g[q] * u2 + M[PK_<5>(1, 2 + q)] * ni;
+#pragma unroll
+                for (int b = 0; b < 3; b++) {
+                    const double cn = g[q] * (M[PK_<5>(0, 2 + b)] * f1 + M[PK_<5>(1, 2 + b)] * f2) + M[PK_<5>(2 + q, 2 + b)] * ni;
+#pragma unroll
+                    for (int j = 0; j < 3; j++)
+                        S[9 * (r - r0) + 3 * b + j][l] = g[b] * (c1 * cmp(F.f1, j) + c2 * cmp(F.f2, j)) + cn * cmp(F.n, j);
+                }
+            }
+            if (r0 < 8) stage_flush<18>(st, a.rec, REC, R_PK + 9 * r0);
+            else { S[9][l] = 0.0; stage_flush<10>(st, a.rec, REC, R_PK + 72); }      // 9 entries and a pad
+        }
+    }
+    double w[4][4];
+    load_w(a.xbar, id0, id1, id2, id3, w);
+    double gmv[4];
+    d3 ft = mk(0, 0, 0);
+    {
+        Fric f;
+        friction_eval(a, is_ee, type, d, B1, P0, P1, P2, P3, id0, id1, id2, id3, f);
+        S[R_D][l] = rec_code(a, cid, 9);
+        fric_fields(f, nside0, w, [&](int k, double v) { S[k][l] = v; });
+        stage_flush<R_Z>(st, a.rec, REC, 0);
+        tk_fields(f, [&](int k, double v) { S[k][l] = v; });
+        stage_flush<TKN>(st, a.tk, TKN, 0);
+        if (valid) a.lam[cid] = f.lam;
+        gmv[0] = f.gm0; gmv[1] = f.gm1; gmv[2] = f.gm2; gmv[3] = f.gm3;
+        if (f.on) {
+            const double t0 = f.fs * f.u0, t1 = f.fs * f.u1;
+            ft = mk(t0 * f.c0.x + t1 * f.c1.x, t0 * f.c0.y + t1 * f.c1.y, t0 * f.c0.z + t1 * f.c1.z);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int al = 0; al < 4; al++) {
+                double zz = 0.0;
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if ((k < nside0) == (s == 0)) zz += kHel[q][k] * w[k][al];
+                S[8 * q + 4 * s + al][l] = zz;
+            }
+    stage_flush<24>(st, a.rec, REC, R_Z);
+    const double gs = 2.0 * B1 * F.delta;
+    d3 gv[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const double g = gs * F.gam[k];
+        gv[k] = mk(g * F.n.x + gmv[k] * ft.x, g * F.n.y + gmv[k] * ft.y, g * F.n.z + gmv[k] * ft.z);
+    }
+    grad_fields(nside0, w, gv, [&](int k, double v) { S[k - R_GRAD][l] = v; });
+    stage_flush<24>(st, a.rec, REC, R_GRAD);
 }
 
 // record fields other than PK of 3-point contacts, one thread each
@@ -1136,12 +1225,14 @@ __device__ __forceinline__ void contact_slices(const WorldArgs& a) {
     for (int p0 = (blockIdx.x * 4 + wv) * 64; p0 < cnt; p0 += gridDim.x * 256) {
         const int p = min(p0 + st.lane, cnt - 1);
         st.nvalid = min(64, cnt - p0);
-        st.cid = a.list[CLS == 1 ? p : total - 1 - p];
+        st.cid = CLS == 3 ? a.list3[p] : a.list[CLS == 1 ? p : total - 1 - p];
         if (CLS == 1) contact_small(a, st, p0 + st.lane < cnt);
+        else if (CLS == 3) contact_plane(a, st, p0 + st.lane < cnt);
         else scalars_c2(a, st, p0 + st.lane < cnt);
     }
 }
 __global__ __launch_bounds__(256) void k_contact_scalars2(WorldArgs a) { contact_slices<2>(a); }
+__global__ __launch_bounds__(256, 2) void k_contact_plane(WorldArgs a) { contact_slices<3>(a); }
 __global__ __launch_bounds__(64) void k_contact_pk2(WorldArgs a) {
     const int total = a.n_pt + a.n_ee;
     const int cnt = a.counts[1];
@@ -1211,7 +1302,7 @@ void contact_terms(World& w) {
     const size_t nn = (size_t)std::max(n, 1);
     w.crec.reserve(REC * nn);
     w.ctype.reserve(nn); w.cdist.reserve(nn); w.ccls.reserve(nn); w.clist.reserve(nn); w.clist3.reserve(nn);
-    w.ccount.reserve(4);
+    w.ccount.reserve(5);
     w.ctk.reserve(TKN * nn);
     w.clam.reserve(nn);
     // the contact set is final here: the assembly's pair structure, which
@@ -1219,8 +1310,8 @@ void contact_terms(World& w) {
     // below, after the contact kernels)
     if (!w.ev_asm_fork) ADB_HIP(hipEventCreateWithFlags(&w.ev_asm_fork, hipEventDisableTiming));
     ADB_HIP(hipEventRecord(w.ev_asm_fork, w.stream));
-    // class counts [0, 3) (entry 3, the chunk count, belongs to the assembly)
-    ADB_HIP(hipMemsetAsync(w.ccount.p, 0, 3 * sizeof(int), w.stream));
+    // class counts [0, 4) (entry 4, the chunk count, belongs to the assembly)
+    ADB_HIP(hipMemsetAsync(w.ccount.p, 0, 4 * sizeof(int), w.stream));
     if (n > 0) {
         WorldArgs a;
         a.kp = make_kp(w.P);
@@ -1240,7 +1331,7 @@ void contact_terms(World& w) {
         }
         const int* snap = prof_snapshot(w, w.ccount.p);
         {
-            // 4-point contacts on the side stream (four 64-lane workgroups per CU,
+            // mollified edge pairs on the side stream (four 64-lane workgroups per CU,
             // one wave per SIMD, FP64-VALU-bound): they overlap the 2- and 3-point
             // kernels and the assembly's sort; the assembly waits for them
             // before its reduction
@@ -1254,7 +1345,7 @@ void contact_terms(World& w) {
             ADB_HIP(hipStreamWaitEvent(w.stream2, w.ev_side[0], 0));
             {
                 ProfScope ps(w, PK_CONTACT_GROUP, 0.0, w.stream2);
-                ps.counts(snap, 0.0, 0.0, 1608.0, 0.0);
+                ps.counts(snap, 0.0, 0.0, 0.0, 1608.0);
                 // the class count is on the device: grids sized for the worst case, grid-stride loops
                 hipLaunchKernelGGL(k_contact_c3r, dim3(std::min((C3_ROLES * n + 255) / 256, 16 * w.num_cu)), dim3(256), 0,
                                    w.stream2, a);
@@ -1269,10 +1360,13 @@ void contact_terms(World& w) {
             // scattered loads and stores); they write disjoint record fields
             ADB_HIP(hipStreamWaitEvent(w.stream3, w.ev_side[0], 0));
             {
-                // per 3-point contact: ids, 4 points, type and distance in; PK (36 doubles) out
+                // per 3-point contact: ids, 4 points, type and distance in; PK (36 doubles)
+                // out; per 4-point contact the whole record (147 doubles) and its inputs
                 ProfScope ps(w, PK_CONTACT_PK, 0.0, w.stream3);
-                ps.counts(snap, 0.0, 440.0, 0.0, 0.0);
+                ps.counts(snap, 0.0, 440.0, 1608.0, 0.0);
                 hipLaunchKernelGGL(k_contact_pk2, dim3(std::min((n + 63) / 64, 16 * w.num_cu)), dim3(64), 0, w.stream3, a);
+                ADB_HIP(hipGetLastError());
+                hipLaunchKernelGGL(k_contact_plane, dim3(std::min((n + 255) / 256, 4 * w.num_cu)), dim3(256), 0, w.stream3, a);
                 ADB_HIP(hipGetLastError());
             }
             ADB_HIP(hipEventRecord(w.ev_pk, w.stream3));

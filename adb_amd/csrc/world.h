@@ -75,7 +75,7 @@ struct Prof {
     bool on = false;
     // bytes of a launch = bytes + sum_i per[i] * snap[i], where snap points to
     // a pinned host copy of device counters taken on the stream before the launch
-    struct Rec { int k; hipEvent_t a, b; double bytes; const int* snap; double per[4]; double flops; };
+    struct Rec { int k; hipEvent_t a, b; double bytes; const int* snap; double per[5]; double flops; };
     std::vector<Rec> pending;
     std::vector<hipEvent_t> pool;
     int* snap = nullptr;             // pinned host ring of counter snapshots
@@ -170,7 +170,7 @@ struct World {
     DBuf<double> cdist;              // squared distance per contact
     DBuf<int> clist;                 // class 1 from the front, class 2 from the back
     DBuf<int> clist3;                // class 3 contacts
-    DBuf<int> ccount;                // 4 counters: class 1, 2, 3 sizes
+    DBuf<int> ccount;                // class 1..4 sizes, chunk count
     DBuf<double> ctk;                // TKN per PT/EE contact: lagged friction basis (see TKN)
     DBuf<double> clam;               // 1 per PT/EE contact
     DBuf<double> vgK;                // 12 per VG contact: K (3x3 col-major) + gx (3)
@@ -278,8 +278,10 @@ constexpr int SRED_N = 4;   // per-scene sum slots
 struct ProfScope {
     World& w; int k; double bytes; hipEvent_t a = nullptr; hipStream_t st;
     double flops = 0.0;               // the launch's counted FP64 operations, when known
-    const int* snap = nullptr; double per[4] = {0, 0, 0, 0};
-    void counts(const int* s, double p0, double p1, double p2, double p3) { snap = s; per[0] = p0; per[1] = p1; per[2] = p2; per[3] = p3; }
+    const int* snap = nullptr; double per[5] = {0, 0, 0, 0, 0};
+    void counts(const int* s, double p0, double p1, double p2, double p3, double p4 = 0.0) {
+        snap = s; per[0] = p0; per[1] = p1; per[2] = p2; per[3] = p3; per[4] = p4;
+    }
     ProfScope(World& w_, int k_, double bytes_, hipStream_t s = nullptr) : w(w_), k(k_), bytes(bytes_), st(s ? s : w_.stream) {
         if (!w.prof.on) return;
         a = get();
@@ -289,7 +291,7 @@ struct ProfScope {
         if (!w.prof.on || !a) return;
         hipEvent_t b = get();
         (void)hipEventRecord(b, st);
-        w.prof.pending.push_back({k, a, b, bytes, snap, {per[0], per[1], per[2], per[3]}, flops});
+        w.prof.pending.push_back({k, a, b, bytes, snap, {per[0], per[1], per[2], per[3], per[4]}, flops});
     }
     hipEvent_t get() {
         if (!w.prof.pool.empty()) { hipEvent_t e = w.prof.pool.back(); w.prof.pool.pop_back(); return e; }

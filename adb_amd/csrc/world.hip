@@ -718,7 +718,7 @@ void prof_flush(World& w) {
         ADB_HIP(hipEventElapsedTime(&ms, r.a, r.b));
         w.prof.ms[r.k] += ms;
         double bytes = r.bytes;
-        if (r.snap) for (int i = 0; i < 4; i++) bytes += r.per[i] * (double)r.snap[i];
+        if (r.snap) for (int i = 0; i < 5; i++) bytes += r.per[i] * (double)r.snap[i];
         w.prof.bytes[r.k] += bytes;
         w.prof.flops[r.k] += r.flops;
         w.prof.count[r.k] += 1;
@@ -731,13 +731,13 @@ void prof_flush(World& w) {
 const int* prof_snapshot(World& w, const int* dev_counts) {
     if (!w.prof.on) return nullptr;
     if (!w.prof.snap) {
-        ADB_HIP(hipHostMalloc((void**)&w.prof.snap, 4 * 8192 * sizeof(int), hipHostMallocDefault));
-        w.prof.snap_cap = 4 * 8192;
+        ADB_HIP(hipHostMalloc((void**)&w.prof.snap, 5 * 8192 * sizeof(int), hipHostMallocDefault));
+        w.prof.snap_cap = 5 * 8192;
     }
-    if (w.prof.snap_used + 4 > w.prof.snap_cap) prof_flush(w);
+    if (w.prof.snap_used + 5 > w.prof.snap_cap) prof_flush(w);
     int* dst = w.prof.snap + w.prof.snap_used;
-    w.prof.snap_used += 4;
-    ADB_HIP(hipMemcpyAsync(dst, dev_counts, 4 * sizeof(int), hipMemcpyDeviceToHost, w.stream));
+    w.prof.snap_used += 5;
+    ADB_HIP(hipMemcpyAsync(dst, dev_counts, 5 * sizeof(int), hipMemcpyDeviceToHost, w.stream));
     return dst;
 }
 } // namespace adb
