@@ -48,7 +48,9 @@ __global__ void k_inertia(int B, double dt, double kap, double ga0, double ga1, 
         return;
     }
     const double* Q = q + 12 * (size_t)b;
-    const d3 a[4] = {ld3(Q), ld3(Q + 3), ld3(Q + 6), ld3(Q + 9)};
+    // columns of q by address: a private array indexed per lane would go
+    // through scratch memory (27 000 bodies 111 -> 43 us)
+    auto a = [&](int i) { return ld3(Q + 3 * i); };
     const double m = mass[b], ic = Ic[b];
     if (e < 12) {
         double go = 0.0;
@@ -56,8 +58,8 @@ __global__ void k_inertia(int B, double dt, double kap, double ga0, double ga1, 
         if (i > 0) {
             double s0 = 0, s1 = 0, s2 = 0;
             for (int j = 1; j < 4; j++) {
-                double s = dot(a[i], a[j]) - (i == j ? 1.0 : 0.0);
-                s0 += s * a[j].x; s1 += s * a[j].y; s2 += s * a[j].z;
+                double s = dot(a(i), a(j)) - (i == j ? 1.0 : 0.0);
+                s0 += s * a(j).x; s1 += s * a(j).y; s2 += s * a(j).z;
             }
             go = 4 * kap * (r == 0 ? s0 : (r == 1 ? s1 : s2));
         }
@@ -69,12 +71,13 @@ __global__ void k_inertia(int B, double dt, double kap, double ga0, double ga1, 
     // H[(3 j + c) * 12 + 3 i + r]
     const int j = col / 3, c = col % 3, i = row / 3, r = row % 3;
     if (i >= 1 && j >= 1) {
+        const d3 ai = a(i), aj = a(j);
         double h;
         if (i == j) {
-            h = 2 * cmp(a[i], r) * cmp(a[i], c) + (r == c ? dot(a[i], a[i]) - 1 : 0.0);
-            for (int k = 1; k < 4; k++) if (k != i) h += cmp(a[k], r) * cmp(a[k], c);
+            h = 2 * Q[3 * i + r] * Q[3 * i + c] + (r == c ? dot(ai, ai) - 1 : 0.0);
+            for (int k = 1; k < 4; k++) if (k != i) h += Q[3 * k + r] * Q[3 * k + c];
         } else {
-            h = (r == c ? dot(a[j], a[i]) : 0.0) + cmp(a[j], r) * cmp(a[i], c);
+            h = (r == c ? dot(aj, ai) : 0.0) + Q[3 * j + r] * Q[3 * i + c];
         }
         hv += h * 4 * kap * dt * dt;
     }
@@ -761,7 +764,39 @@ __device__ __forceinline__ void group_blocks(int lane, int nl, int m, const int*
         blk[e] = k;
     }
 }
-__global__ __launch_bounds__(256) void k_group_inv(const int* __restrict__ list, int nb8, int n4,
+// The inverse of a single body's block: 12 lanes, lane r holding row r (of the
+// upper triangle mirrored), the pivot rows by lane reads; the operations of
+// sweep12 in their order.  A wavefront per body in the block sweep left 57 of
+// 64 lanes without a tile (27 000 bodies, most of them single: 212 -> 69 us).
+__device__ __forceinline__ void invert_single(bool on, int r, int row0, const double* __restrict__ H, double* __restrict__ out) {
+    double v[12];
+#pragma unroll
+    for (int c = 0; c < 12; c++) v[c] = on ? H[c >= r ? 12 * c + r : 12 * r + c] : (c == r ? 1.0 : 0.0);
+    bool pd = true;
+#pragma unroll
+    for (int k = 0; k < 12; k++) {
+        const double d = __shfl(v[k], row0 + k);
+        pd = pd && d > 0.0 && d < INFINITY;
+        const double inv = 1.0 / d, ci = v[k];
+#pragma unroll
+        for (int c = 0; c < 12; c++) {
+            if (c == k) continue;
+            const double w = __shfl(v[c], row0 + k) * inv;
+            v[c] = r == k ? w : v[c] - ci * w;
+        }
+        v[k] = r == k ? -inv : ci * inv;
+    }
+    if (!on) return;
+#pragma unroll
+    for (int c = 0; c < 12; c++)
+        if (c >= r) {
+            // not positive definite: the inverse of the diagonal
+            const double x = pd ? -v[c] : (c == r ? 1.0 / (H[13 * r] > 0.0 ? H[13 * r] : 1.0) : 0.0);
+            out[12 * c + r] = x;
+            out[12 * r + c] = x;
+        }
+}
+__global__ __launch_bounds__(256) void k_group_inv(const int* __restrict__ list, int nb8, int n4, int n1, const int* __restrict__ diag_blk,
                                                    const int* __restrict__ grp_off, const int* __restrict__ grp_body,
                                                    const long long* __restrict__ grp_moff, const int* __restrict__ row_ptr,
                                                    const int* __restrict__ col_idx, const double* __restrict__ Hval,
@@ -779,7 +814,7 @@ __global__ __launch_bounds__(256) void k_group_inv(const int* __restrict__ list,
         group_blocks(t, 256, m, bod[0], row_ptr, col_idx, blk[0]);
         __syncthreads();
         group_bsweep<96, 256, GI_LD>(t, m, blk[0], Hval, Ginv + grp_moff[g], sm, true);
-    } else {
+    } else if ((int)blockIdx.x < nb8 + (n4 + 3) / 4) {
         const int q = 4 * ((int)blockIdx.x - nb8) + wv;           // one group per wavefront
         if (q >= n4) return;                                       // whole wavefront: no block barrier below
         const int g = list[nb8 + q];
@@ -789,6 +824,12 @@ __global__ __launch_bounds__(256) void k_group_inv(const int* __restrict__ list,
         group_blocks(ln, 64, m, bod[wv], row_ptr, col_idx, blk[wv]);
         gi_sync(false);
         group_bsweep<48, 64, GI_LD4>(ln, m, blk[wv], Hval, Ginv + grp_moff[g], sm + wv * GI_LDS4, false);
+    } else {
+        // five single bodies per wavefront
+        const int s = 20 * ((int)blockIdx.x - nb8 - (n4 + 3) / 4) + 5 * wv + ln / 12;
+        const bool on = ln < 60 && s < n1;
+        const int g = list[nb8 + n4 + (on ? s : 0)];
+        invert_single(on, ln % 12, min(ln / 12, 4) * 12, Hval + 144 * (size_t)diag_blk[grp_body[grp_off[g]]], Ginv + grp_moff[g]);
     }
 }
 
@@ -1259,10 +1300,10 @@ void assemble_system(World& w) {
             ps.flops = fl;
         }
         static_assert(GMAX == 8, "size classes 5..8 and 1..4");
-        const int n4 = w.n_glist[1] + w.n_glist[2];
-        const int nb = w.n_glist[0] + (n4 + 3) / 4;
+        const int n4 = w.n_glist[1], n1 = w.n_glist[2];
+        const int nb = w.n_glist[0] + (n4 + 3) / 4 + (n1 + 19) / 20;
         if (nb > 0)
-            hipLaunchKernelGGL(k_group_inv, dim3(nb), dim3(256), 0, w.stream, w.glist, w.n_glist[0], n4, w.grp_off,
+            hipLaunchKernelGGL(k_group_inv, dim3(nb), dim3(256), 0, w.stream, w.glist, w.n_glist[0], n4, n1, w.diag_blk.p, w.grp_off,
                                w.grp_body, w.grp_moff, w.row_ptr.p, w.col_idx.p, w.Hval.p, w.Ginv.p);
         ADB_HIP(hipGetLastError());
         tree_factor(w);
