@@ -57,11 +57,11 @@ struct KParams {
 };
 
 // ---------------------------------------------------------------- barrier Hessian column
-// Contact geometry and barrier scalars, computed redundantly by every lane of
-// the group (no private arrays indexed by lane-dependent values).
+// Geometry and barrier scalars of a mollified edge pair (no private arrays
+// indexed by lane-dependent values).
 struct Geo {
     d3 p0, p1, p2, p3;
-    int is_ee, type;
+    int type;
     double d, B0, B1, B2;
     double m, m1, m2;       // EE mollifier m(x) and dm/dx, d2m/dx2
     RedMap map;
@@ -73,44 +73,30 @@ __device__ __forceinline__ void geo_init(Geo& G, const KParams& kp) {
     const double dh = kp.d_hat, ka = kp.kappa;
     G.B1 = barrier_d1(G.d, dh, ka);
     G.B2 = barrier_d2(G.d, dh, ka);
-    G.B0 = G.is_ee ? barrier(G.d, dh, ka) : 0.0;
-    G.map = G.is_ee ? ee_map(G.type) : pt_map(G.type);
+    G.B0 = barrier(G.d, dh, ka);
+    G.map = ee_map(G.type);
     d3 r0 = mk(0, 0, 0), r1 = mk(0, 0, 0), r2 = mk(0, 0, 0);
     const d3 p0 = G.p0, p1 = G.p1, p2 = G.p2, p3 = G.p3;
-    if (!G.is_ee) {
-        switch (G.type) {
-        case P_T0: r0 = p0 - p1; break;
-        case P_T1: r0 = p0 - p2; break;
-        case P_T2: r0 = p0 - p3; break;
-        case P_E0: r0 = p1 - p0; r1 = p2 - p0; break;
-        case P_E1: r0 = p2 - p0; r1 = p3 - p0; break;
-        case P_E2: r0 = p3 - p0; r1 = p1 - p0; break;
-        default:   r0 = p0 - p1; r1 = p2 - p1; r2 = p3 - p1; break;
-        }
-    } else {
-        switch (G.type) {
-        case EA0_EB0: r0 = p0 - p2; break;
-        case EA0_EB1: r0 = p0 - p3; break;
-        case EA1_EB0: r0 = p1 - p2; break;
-        case EA1_EB1: r0 = p1 - p3; break;
-        case EA_EB0:  r0 = p0 - p2; r1 = p1 - p2; break;
-        case EA_EB1:  r0 = p0 - p3; r1 = p1 - p3; break;
-        case EA0_EB:  r0 = p2 - p0; r1 = p3 - p0; break;
-        case EA1_EB:  r0 = p2 - p1; r1 = p3 - p1; break;
-        default:      r0 = p2 - p0; r1 = p1 - p0; r2 = p3 - p2; break;
-        }
+    switch (G.type) {
+    case EA0_EB0: r0 = p0 - p2; break;
+    case EA0_EB1: r0 = p0 - p3; break;
+    case EA1_EB0: r0 = p1 - p2; break;
+    case EA1_EB1: r0 = p1 - p3; break;
+    case EA_EB0:  r0 = p0 - p2; r1 = p1 - p2; break;
+    case EA_EB1:  r0 = p0 - p3; r1 = p1 - p3; break;
+    case EA0_EB:  r0 = p2 - p0; r1 = p3 - p0; break;
+    case EA1_EB:  r0 = p2 - p1; r1 = p3 - p1; break;
+    default:      r0 = p2 - p0; r1 = p1 - p0; r2 = p3 - p2; break;
     }
     G.rd.init(G.map.kind, r0, r1, r2);
     G.m = 1.0; G.m1 = 0.0; G.m2 = 0.0;
-    if (G.is_ee) {
-        const double eps = kp.eps_x * sqn(p0 - p1) * sqn(p2 - p3);
-        G.mc.init(p1 - p0, p3 - p2);
-        const double x = G.mc.value();
-        if (x < eps) {
-            G.m = (-x / eps + 2) * x / eps;
-            G.m1 = 2.0 / eps - 2.0 * x / (eps * eps);
-            G.m2 = -2.0 / (eps * eps);
-        }
+    const double eps = kp.eps_x * sqn(p0 - p1) * sqn(p2 - p3);
+    G.mc.init(p1 - p0, p3 - p2);
+    const double x = G.mc.value();
+    if (x < eps) {
+        G.m = (-x / eps + 2) * x / eps;
+        G.m1 = 2.0 / eps - 2.0 * x / (eps * eps);
+        G.m2 = -2.0 / (eps * eps);
     }
 }
 // point-space gradient entry (k, i) of d, and of the mollifier
@@ -132,7 +118,7 @@ __device__ __forceinline__ double grad_m(const Geo& G, int k, int i) {
 __device__ __forceinline__ double barrier_grad(const Geo& G, int j) {
     const int l = j / 3, c = j % 3;
     const double gdj = grad_d(G, l, c);
-    return G.is_ee ? G.m * gdj * G.B1 + grad_m(G, l, c) * G.B0 : gdj * G.B1;
+    return G.m * gdj * G.B1 + grad_m(G, l, c) * G.B0;
 }
 
 // ---------------------------------------------------------------- friction setup
@@ -776,7 +762,7 @@ struct C3Ctx {
 __device__ __forceinline__ void c3_setup(const WorldArgs& a, int cid, C3Ctx& x) {
     x.R = a.rec + REC * (size_t)cid;
     Geo& G = x.G;
-    G.is_ee = contact_ids(a, cid, x.id0, x.id1, x.id2, x.id3);
+    contact_ids(a, cid, x.id0, x.id1, x.id2, x.id3);
     G.p0 = ld3(a.X + 3 * (size_t)x.id0); G.p1 = ld3(a.X + 3 * (size_t)x.id1);
     G.p2 = ld3(a.X + 3 * (size_t)x.id2); G.p3 = ld3(a.X + 3 * (size_t)x.id3);
     G.type = a.ctype[cid]; G.d = a.cdist[cid];
@@ -818,7 +804,7 @@ __device__ __forceinline__ void c3_kbuild(const C3Ctx& x, int role) {
                         for (int b = 0; b < 3; b++) K[q][b] += C[q][m] * C[b][n] * Mv;
                 }
             }
-        if (G.is_ee) {
+        {
             double gdi[3], gdj[3], gxi[3], gxj[3];
 #pragma unroll
             for (int q = 0; q < 3; q++) {
@@ -862,7 +848,7 @@ __device__ __forceinline__ void c3_fields(const WorldArgs& a, int cid, const C3C
     const Geo& G = x.G;
     double* R = x.R;
     const int id0 = x.id0, id1 = x.id1, id2 = x.id2, id3 = x.id3;
-    const int nside0 = G.is_ee ? 2 : 1;
+    const int nside0 = 2;
     double w[4][4];
     load_w(a.xbar, id0, id1, id2, id3, w);
 #pragma unroll
@@ -878,7 +864,7 @@ __device__ __forceinline__ void c3_fields(const WorldArgs& a, int cid, const C3C
                 R[R_Z + 8 * q + 4 * s + al] = zz;
             }
     Fric f;
-    friction_eval(a, G.is_ee, G.type, G.d, G.B1, G.p0, G.p1, G.p2, G.p3, id0, id1, id2, id3, f);
+    friction_eval(a, 1, G.type, G.d, G.B1, G.p0, G.p1, G.p2, G.p3, id0, id1, id2, id3, f);
     write_fric(a, cid, nside0, f, w);
     const double gmv[4] = {f.gm0, f.gm1, f.gm2, f.gm3};
     d3 gv[4];

@@ -47,15 +47,10 @@ constexpr double JACOBI_TOL = 1e-24;
 // such entries add at most 36e-28 |A|_F^2 to the off-diagonal sum, far below
 // the stop test, and late sweeps then cost little
 constexpr double JACOBI_SKIP = 1e-14;
-// Reciprocal and reciprocal square root from the hardware approximations,
-// each refined by two Newton steps (each step doubles the correct bits).
-// The Jacobi rotation parameters need no correct rounding, and this chain is
-// several times shorter than IEEE division and square root.
-__device__ __forceinline__ double rcp_r(double x) {
-    double y = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, y, 1.0); y = fma(y, e, y);
-    e = fma(-x, y, 1.0); return fma(y, e, y);
-}
+// Reciprocal square root from the hardware approximation, refined by two
+// Newton steps (each doubles the correct bits).  The Jacobi rotation parameters
+// need no correct rounding, and this chain is several times shorter than IEEE
+// division and square root.
 __device__ __forceinline__ double rsq_r(double x) {
     double y = __builtin_amdgcn_rsq(x);
     const double h = 0.5 * x;
