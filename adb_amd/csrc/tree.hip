@@ -6,6 +6,14 @@
 // Two chains of 32 tori (5 rounds) 90 us and 100 rows of 100 cards (7 rounds)
 // 206 us, against 73 and 264 us for the explicit inverses of groups of 8 that
 // left 160 and 124 PCG iterations (9 and 32 us each).
+//
+// A pivot that is not positive and finite (a matrix that is not positive
+// definite, or a Schur complement lost to rounding between contacts 1e16 times
+// stiffer than the inertia) gives way to the matrix's own diagonal entry there:
+// the factors are those of the matrix with that entry raised, a change of rank
+// one that costs PCG a few iterations, whatever the component's size.  With the
+// inverse diagonal in place of the whole factor a column of 40 cubes with one
+// such contact ran to the limit of 2000.
 #include "dmath.h"
 #include "tree.h"
 #include "world.h"
@@ -56,7 +64,6 @@ struct TreeArgs {
 };
 constexpr int TREE_T = 512, TREE_U = 4;
 __global__ __launch_bounds__(TREE_T) void k_tree_factor(TreeArgs a) {
-    __shared__ int bad;
     const int g = a.list[blockIdx.x];
     // the table, but for the contribution lists, in LDS: its indices are links
     // of every chain of loads below
@@ -71,7 +78,6 @@ __global__ __launch_bounds__(TREE_T) void k_tree_factor(TreeArgs a) {
     double* F = a.Ginv + a.grp_moff[g];
     double* V = F + 144 * (size_t)t.n;
     const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
-    if (threadIdx.x == 0) bad = 0;
     for (int l = 0; l < t.nlev; l++) {
         const int p0 = t.lev[l], np = t.lev[l + 1] - p0, e0 = t.up[p0], ne = t.up[p0 + np] - e0;
         // D_j and A_ij = H_ij - sum V V^T of the round's columns, TREE_U blocks
@@ -114,12 +120,14 @@ __global__ __launch_bounds__(TREE_T) void k_tree_factor(TreeArgs a) {
                 v[c] = on ? F[144 * (size_t)j + 12 * c + r] : (c == r ? 1.0 : 0.0);
                 x[c] = c == r ? 1.0 : 0.0;
             }
-            bool pd = true;
 #pragma unroll
             for (int k = 0; k < 12; k++) {
                 const int row = min(12 * m, 48);
-                const double d = __shfl(v[k], row + k);
-                pd = pd && d > 0.0 && d < INFINITY;
+                double d = __shfl(v[k], row + k);
+                if (!(d > 0.0 && d < INFINITY)) {
+                    d = on ? fabs(a.Hval[144 * (size_t)a.diag_blk[t.body[j]] + 13 * k]) : 1.0;
+                    if (!(d > 0.0 && d < INFINITY)) d = 1.0;
+                }
                 const double inv = rsq2(d), f = v[k] * inv;            // L_rk
                 v[k] = f;
 #pragma unroll
@@ -130,7 +138,6 @@ __global__ __launch_bounds__(TREE_T) void k_tree_factor(TreeArgs a) {
                     x[c] = r == k ? y : (r > k ? x[c] - f * y : x[c]);
                 }
             }
-            if (on && !pd) bad = 1;
             // row r of L^-1, and row r of L as column r above the diagonal
             if (on)
 #pragma unroll
@@ -140,7 +147,6 @@ __global__ __launch_bounds__(TREE_T) void k_tree_factor(TreeArgs a) {
                 }
         }
         __syncthreads();
-        if (bad) break;
         // V_ij = A_ij L_j^-T by substitution, 12 lanes a block, lane r its row r
         for (int s = wv * 5; s < ne; s += TREE_T / 64 * 5) {
             const int r = lane % 12, e = e0 + s + lane / 12;
@@ -162,18 +168,6 @@ __global__ __launch_bounds__(TREE_T) void k_tree_factor(TreeArgs a) {
         }
         __syncthreads();
     }
-    if (!bad) return;
-    // not positive definite: the inverse of the matrix's diagonal
-    for (int x = threadIdx.x; x < 144 * t.n; x += TREE_T) {
-        const int e = x % 144, i = e % 12;
-        double v = 0.0;
-        if (e / 12 == i) {
-            const double d = a.Hval[144 * (size_t)a.diag_blk[t.body[x / 144]] + 13 * i];
-            v = 1.0 / sqrt(d > 0.0 ? d : 1.0);
-        }
-        F[x] = v;
-    }
-    for (size_t x = threadIdx.x; x < 144 * (size_t)t.ne; x += TREE_T) V[x] = 0.0;
 }
 
 // factors of the tree groups (build_groups queued their tables' upload)
