@@ -872,14 +872,14 @@ static void groups_fetch(World& w, int npb, const int* npd, const int* pack, hip
 }
 // The components of the contact graph of more than TREE_MIN bodies that become one
 // group each (tree.h): hg_tree (a body's component or -1), its table's offset
-// and block count, and h_tree = the group ids (filled by build_groups), then
-// the tables.  Static bodies take no part: their rows have no off-diagonal
-// blocks.
+// and block count, the tables (hg_tabs), and room for the group ids
+// (hg_tree_grp, filled by build_groups).  Static bodies take no part: their
+// rows have no off-diagonal blocks.
 static void plan_trees(World& w, int np, const int* plo, const int* phi) {
     const int B = w.B;
     std::vector<int>&par = w.hg_cpar, &tree = w.hg_tree, &loc = w.hg_loc;
     tree.assign(B, -1);
-    w.hg_tree_tab.clear(); w.hg_tree_ne.clear(); w.h_tree.clear();
+    w.hg_tree_tab.clear(); w.hg_tree_ne.clear(); w.hg_tree_grp.clear();
     w.n_trees = 0;
     // a caller that caps the iterations at a few asks for the truncated solve
     // (and the report that it was), whose iterates are those of the small groups
@@ -938,8 +938,7 @@ static void plan_trees(World& w, int np, const int* plo, const int* phi) {
         w.hg_tree_ne.push_back(tabs[at + 2]);
         w.n_trees++;
     }
-    w.h_tree.assign(w.n_trees, 0);
-    w.h_tree.insert(w.h_tree.end(), tabs.begin(), tabs.end());
+    w.hg_tree_grp.assign(w.n_trees, 0);
 }
 static void build_groups(World& w) {
     wait_event(w, w.ev_pairs);
@@ -1000,7 +999,7 @@ static void build_groups(World& w) {
         const long long n = 12 * (long long)(w.h_grp_off[g + 1] - w.h_grp_off[g]);
         const int tr = tree[w.h_grp_body[w.h_grp_off[g]]];
         w.h_grp_moff[g + 1] = w.h_grp_moff[g] + (tr < 0 ? n * n : TreePlan::doubles((int)(n / 12), w.hg_tree_ne[tr]));
-        if (tr >= 0) w.h_tree[tr] = g;
+        if (tr >= 0) w.hg_tree_grp[tr] = g;
     }
     w.n_groups = G;
     if (w.S > 1) {
@@ -1034,9 +1033,10 @@ static void build_groups(World& w) {
     w.n_glist[2] = (int)w.h_glist.size() - w.n_glist[0] - w.n_glist[1];
     // one upload of all group tables (pinned staging; the previous upload from
     // it has completed before it is rewritten).  Offsets depend on B only (at
-    // most B groups), so the tables' device addresses stay the same from one
-    // Newton iteration to the next (the captured PCG batch is keyed on them).
-    const size_t nll = (size_t)B + 1, nint = (size_t)(B + 1) + B + B + B + 1, total = nll + (nint + 1) / 2;
+    // most B groups, a component's group has more than TREE_MIN bodies), so the
+    // tables' device addresses stay the same from one Newton iteration to the
+    // next (the captured PCG batch is keyed on them).
+    const size_t nll = (size_t)B + 1, nint = (size_t)(B + 1) + B + B + B + 1 + B / (TREE_MIN + 1), total = nll + (nint + 1) / 2;
     if (!w.ev_grp) ADB_HIP(hipEventCreateWithFlags(&w.ev_grp, hipEventDisableTiming));
     wait_event(w, w.ev_grp);
     if (total > w.h_grp_pack_cap) {
@@ -1059,6 +1059,7 @@ static void build_groups(World& w) {
             ht[g] = tr < 0 ? -1 : w.hg_tree_tab[tr];
         }
         hi[4 * B + 1] = G;
+        std::memcpy(hi + 4 * B + 2, w.hg_tree_grp.data(), (size_t)w.n_trees * sizeof(int));
     }
     w.grp_moff = w.grp_pack.p;
     w.grp_off = reinterpret_cast<int*>(w.grp_pack.p + nll);
@@ -1066,17 +1067,18 @@ static void build_groups(World& w) {
     w.glist = w.grp_body + B;
     w.grp_tree = w.glist + B;
     w.grp_n = w.grp_tree + B;
+    w.tree_list = w.grp_n + 1;
     ADB_HIP(hipMemcpyAsync(w.grp_pack.p, w.h_grp_pack, total * sizeof(long long), hipMemcpyHostToDevice, w.stream));
     if (w.n_trees > 0) {
-        // the tree groups' ids, then their tables
-        const size_t nt = w.h_tree.size();
+        // the tree groups' tables, in a buffer that moves only when it grows
+        const size_t nt = w.hg_tabs.size();
         if (nt > w.h_tree_pin_cap) {
             if (w.h_tree_pin) ADB_HIP(hipHostFree(w.h_tree_pin));
             w.h_tree_pin = nullptr;
             w.h_tree_pin_cap = nt + nt / 2;
             ADB_HIP(hipHostMalloc((void**)&w.h_tree_pin, w.h_tree_pin_cap * sizeof(int), hipHostMallocDefault));
         }
-        std::memcpy(w.h_tree_pin, w.h_tree.data(), nt * sizeof(int));
+        std::memcpy(w.h_tree_pin, w.hg_tabs.data(), nt * sizeof(int));
         w.tree_pack.reserve(nt);
         ADB_HIP(hipMemcpyAsync(w.tree_pack.p, w.h_tree_pin, nt * sizeof(int), hipMemcpyHostToDevice, w.stream));
     }
@@ -1294,7 +1296,7 @@ void assemble_system(World& w) {
                 if (w.h_grp_off[g + 1] - w.h_grp_off[g] <= GMAX) fl += group_inv_flops(w.h_grp_off[g + 1] - w.h_grp_off[g]);
             // the trees: block products, substitutions, factors and their inverses
             for (int tr = 0; tr < w.n_trees; tr++) {
-                const int* T = w.h_tree.data() + w.n_trees + w.hg_tree_tab[tr];
+                const int* T = w.hg_tabs.data() + w.hg_tree_tab[tr];
                 fl += 3456.0 * (T[2] + T[3]) + 1728.0 * T[2] + 1152.0 * T[0];
             }
             ps.flops = fl;

@@ -433,7 +433,7 @@ __global__ __launch_bounds__(UPD_T) void k_pcg_update(int kloc, int nbS, Groups 
 static Groups groups_of(World& w) {
     Groups G;
     G.off = w.grp_off; G.body = w.grp_body; G.moff = w.grp_moff; G.Minv = w.Ginv.p; G.count = w.grp_n;
-    G.tree = w.grp_tree; G.tab = w.tree_pack.p + w.n_trees;
+    G.tree = w.grp_tree; G.tab = w.tree_pack.p;
     return G;
 }
 
@@ -497,6 +497,32 @@ static void enqueue_batch(World& w, int nb, bool prof) {
     hipLaunchKernelGGL(k_pcg_advance, dim3(1), dim3(64), 0, w.stream, w.scal.p, nb);
 }
 
+// A whole batch as a graph, captured when one is first needed and again when a
+// buffer it was captured with has moved.  Contact components come and go
+// from one iteration to the next, so their number is no part of the key.
+static void launch_batch_graph(World& w, int batch) {
+    const bool trees = w.n_trees > 0;
+    World::PcgGraph& gr = w.pcg_graph[trees];
+    const void* key[] = {w.row_ptr.p, w.col_idx.p, w.Hval.p, w.Ginv.p, w.pcg_xo, w.pcg_r.p, w.pcg_z.p, w.pcg_p.p,
+                         w.pcg_p2.p, w.pcg_Ap.p, w.partial.p, w.scal.p, w.grp_off, w.grp_body, w.grp_moff,
+                         w.grp_n, w.sc_goff.p, w.pcg_sbb.p, trees ? w.tree_pack.p : nullptr};
+    static_assert(sizeof key / sizeof key[0] == World::PCG_GRAPH_KEYS, "graph key size");
+    bool same = gr.exec != nullptr && gr.batch == batch;
+    for (int i = 0; i < World::PCG_GRAPH_KEYS; i++) same = same && gr.key[i] == key[i];
+    if (!same) {
+        if (gr.exec) { ADB_HIP(hipGraphExecDestroy(gr.exec)); gr.exec = nullptr; }
+        hipGraph_t g;
+        ADB_HIP(hipStreamBeginCapture(w.stream, hipStreamCaptureModeThreadLocal));
+        enqueue_batch(w, batch, false);
+        ADB_HIP(hipStreamEndCapture(w.stream, &g));
+        ADB_HIP(hipGraphInstantiate(&gr.exec, g, nullptr, nullptr, 0));
+        ADB_HIP(hipGraphDestroy(g));
+        for (int i = 0; i < World::PCG_GRAPH_KEYS; i++) gr.key[i] = key[i];
+        gr.batch = batch;
+    }
+    ADB_HIP(hipGraphLaunch(gr.exec, w.stream));
+}
+
 int pcg_solve(World& w, double* dq_out, int* iters, const std::function<void()>& after, bool* after_valid) {
     if (after_valid) *after_valid = false;
     const int B = w.B, n = 12 * B;
@@ -515,30 +541,9 @@ int pcg_solve(World& w, double* dq_out, int* iters, const std::function<void()>&
         launch_scene_stop(w, 1);
         ADB_HIP(hipGetLastError());
     }
-    // the batch graph is captured once per set of buffer addresses (not while
-    // per-kernel profiling is on, nor with ADB_PCG_GRAPH=0 for tools that do
-    // not support graph capture)
+    // batches go out as a captured graph, but not while per-kernel profiling is
+    // on, nor with ADB_PCG_GRAPH=0 (for tools that do not support graph capture)
     const bool use_graph = !w.prof.on && w.use_graphs;
-    if (use_graph) {
-        const void* key[] = {w.row_ptr.p, w.col_idx.p, w.Hval.p, w.Ginv.p, w.pcg_xo, w.pcg_r.p, w.pcg_z.p, w.pcg_p.p,
-                             w.pcg_p2.p, w.pcg_Ap.p, w.partial.p, w.scal.p, w.grp_off, w.grp_body, w.grp_moff,
-                             w.grp_n, w.sc_goff.p, w.pcg_sbb.p, w.n_trees ? w.tree_pack.p + w.n_trees : nullptr};
-        static_assert(sizeof key / sizeof key[0] == World::PCG_GRAPH_KEYS, "graph key size");
-        const int BATCH = w.tune.pcg_batch;
-        bool same = w.pcg_graph != nullptr && w.pcg_graph_batch == BATCH;
-        for (int i = 0; i < World::PCG_GRAPH_KEYS; i++) same = same && w.pcg_graph_key[i] == key[i];
-        if (!same) {
-            if (w.pcg_graph) { ADB_HIP(hipGraphExecDestroy(w.pcg_graph)); w.pcg_graph = nullptr; }
-            hipGraph_t g;
-            ADB_HIP(hipStreamBeginCapture(w.stream, hipStreamCaptureModeThreadLocal));
-            enqueue_batch(w, BATCH, false);
-            ADB_HIP(hipStreamEndCapture(w.stream, &g));
-            ADB_HIP(hipGraphInstantiate(&w.pcg_graph, g, nullptr, nullptr, 0));
-            ADB_HIP(hipGraphDestroy(g));
-            for (int i = 0; i < World::PCG_GRAPH_KEYS; i++) w.pcg_graph_key[i] = key[i];
-            w.pcg_graph_batch = BATCH;
-        }
-    }
     const int BATCH = w.tune.pcg_batch;
     int it = 0, slot = 0;
     bool have_prev = false;
@@ -575,7 +580,7 @@ int pcg_solve(World& w, double* dq_out, int* iters, const std::function<void()>&
     while (!done && it < max_it) {
         int nb = std::min(BATCH, max_it - it);
         if (pred > 0 && it + BATCH > pred - 8) nb = std::min(nb, 4);
-        if (use_graph && nb == BATCH) ADB_HIP(hipGraphLaunch(w.pcg_graph, w.stream));
+        if (use_graph && nb == BATCH) launch_batch_graph(w, BATCH);
         else enqueue_batch(w, nb, w.prof.on);
         it += nb;
         ADB_HIP(hipGetLastError());

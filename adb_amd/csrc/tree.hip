@@ -174,7 +174,7 @@ __global__ __launch_bounds__(TREE_T) void k_tree_factor(TreeArgs a) {
 void tree_factor(World& w) {
     if (w.n_trees == 0) return;
     TreeArgs a;
-    a.list = w.tree_pack.p; a.tab = w.tree_pack.p + w.n_trees;
+    a.list = w.tree_list; a.tab = w.tree_pack.p;
     a.grp_tree = w.grp_tree; a.grp_moff = w.grp_moff;
     a.pair_up = w.pair_up.p; a.pair_low = w.pair_low.p; a.diag_blk = w.diag_blk.p;
     a.Hval = w.Hval.p; a.Ginv = w.Ginv.p;

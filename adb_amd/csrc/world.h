@@ -207,12 +207,13 @@ struct World {
     long long* grp_moff = nullptr;
     int *grp_off = nullptr, *grp_body = nullptr, *glist = nullptr, *grp_n = nullptr;
     int* grp_tree = nullptr;         // per group: its table's offset in the tree tables, or -1
-    DBuf<int> tree_pack;             // tree groups' ids (n_trees), then their tables (tree.h)
+    int* tree_list = nullptr;        // the tree groups' ids
+    DBuf<int> tree_pack;             // their tables (tree.h)
     int n_trees = 0;
     int* h_tree_pin = nullptr;
     size_t h_tree_pin_cap = 0;
     TreePlan tree_plan;
-    std::vector<int> h_tree, hg_tree, hg_tree_tab, hg_tree_ne, hg_cpar, hg_ccnt, hg_cid, hg_loc, hg_boff, hg_bods, hg_poff, hg_prs,
+    std::vector<int> hg_tree, hg_tree_grp, hg_tree_tab, hg_tree_ne, hg_cpar, hg_ccnt, hg_cid, hg_loc, hg_boff, hg_bods, hg_poff, hg_prs,
         hg_fill, hg_tabs;
     DBuf<double> Ginv;
     int n_groups = 0;
@@ -234,9 +235,14 @@ struct World {
     hipEvent_t ev_pairs = nullptr;   // their copy is done
     hipEvent_t ev_phase[2] = {nullptr, nullptr};   // contact terms + assembly on the stream: start, end
     bool use_graphs = true;          // ADB_PCG_GRAPH=0 turns graph capture off
-    hipGraphExec_t pcg_graph = nullptr;   // one captured PCG batch
-    static constexpr int PCG_GRAPH_KEYS = 19;
-    const void* pcg_graph_key[PCG_GRAPH_KEYS] = {};   // buffer addresses the graph was captured with
+    // one captured PCG batch per form of the update kernel (without and with
+    // tree groups): a step in which contacts come and go alternates between them
+    static constexpr int PCG_GRAPH_KEYS = 19, PCG_FORMS = 2;
+    struct PcgGraph {
+        hipGraphExec_t exec = nullptr;
+        int batch = 0;                            // PCG batch size it was captured with
+        const void* key[PCG_GRAPH_KEYS] = {};     // buffer addresses it was captured with
+    } pcg_graph[PCG_FORMS];
     double* h_scal = nullptr;        // pinned host copies of the PCG scalars (2 x 8)
     hipEvent_t pcg_ev[2] = {nullptr, nullptr};
     // ---- energies
@@ -269,7 +275,6 @@ struct World {
     // launch shapes that change how fast a step runs, never its results
     // (adb_set_tuning; adb_amd/autotune.py picks them per workload)
     adb_tuning tune = {1.125, 4, 16};
-    int pcg_graph_batch = 0;              // PCG batch size the graph was captured with
 };
 constexpr int SRED_N = 4;   // per-scene sum slots
 

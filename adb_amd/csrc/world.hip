@@ -584,10 +584,12 @@ static void free_world(World& w) {
     w.prof.pool.clear();
     if (w.prof.snap) (void)hipHostFree(w.prof.snap);
     w.prof.snap = nullptr;
-    if (w.pcg_graph) (void)hipGraphExecDestroy(w.pcg_graph);
-    w.pcg_graph = nullptr;
+    for (auto& g : w.pcg_graph) {
+        if (g.exec) (void)hipGraphExecDestroy(g.exec);
+        g.exec = nullptr;
+    }
     w.grp_pack.free_();
-    w.grp_moff = nullptr; w.grp_off = w.grp_body = w.glist = w.grp_n = w.grp_tree = nullptr;
+    w.grp_moff = nullptr; w.grp_off = w.grp_body = w.glist = w.grp_n = w.grp_tree = w.tree_list = nullptr;
     w.tree_pack.free_();
     if (w.h_tree_pin) (void)hipHostFree(w.h_tree_pin);
     w.h_tree_pin = nullptr; w.h_tree_pin_cap = 0;
