@@ -881,6 +881,8 @@ static void plan_trees(World& w, int np, const int* plo, const int* phi) {
     tree.assign(B, -1);
     w.hg_tree_tab.clear(); w.hg_tree_ne.clear(); w.hg_tree_grp.clear();
     w.n_trees = 0;
+    w.tree_rest = false;
+    w.tree_doubles = 0;
     // a caller that caps the iterations at a few asks for the truncated solve
     // (and the report that it was), whose iterates are those of the small groups
     if (w.P.pcg_max_iter < TREE_MIN_ITER) return;
@@ -936,8 +938,10 @@ static void plan_trees(World& w, int np, const int* plo, const int* phi) {
         for (int x = boff[c]; x < boff[c + 1]; x++) tree[bods[x]] = w.n_trees;
         w.hg_tree_tab.push_back(at);
         w.hg_tree_ne.push_back(tabs[at + 2]);
+        w.tree_doubles += TreePlan::doubles(n, tabs[at + 2]);
         w.n_trees++;
     }
+    for (int b = 0; b < B && !w.tree_rest; b++) w.tree_rest = par[b] == b && cnt[b] > GMAX && tree[b] < 0;
     w.hg_tree_grp.assign(w.n_trees, 0);
 }
 static void build_groups(World& w) {

@@ -210,6 +210,8 @@ struct World {
     int* tree_list = nullptr;        // the tree groups' ids
     DBuf<int> tree_pack;             // their tables (tree.h)
     int n_trees = 0;
+    bool tree_rest = false;          // some other component is spread over several groups
+    long long tree_doubles = 0;      // doubles of their factors
     int* h_tree_pin = nullptr;
     size_t h_tree_pin_cap = 0;
     TreePlan tree_plan;
@@ -227,7 +229,7 @@ struct World {
     // ---- PCG
     DBuf<double> pcg_r, pcg_z, pcg_p, pcg_p2, pcg_Ap, partial, scal;
     double* pcg_xo = nullptr;        // the solve's iterate: the caller's output buffer
-    int pcg_prev_its = 0;            // iterations of the previous solve
+    int pcg_prev_its[3] = {0, 0, 0}; // iterations of the previous solve: whole, tree part, rest
     int* h_pairs = nullptr;          // pinned host copy of the pair count and lists (lo, hi, start)
     size_t h_pairs_cap = 0;
     int h_pairs_n = 0;               // entries per list in h_pairs (the pair count or its bound)
@@ -235,15 +237,16 @@ struct World {
     hipEvent_t ev_pairs = nullptr;   // their copy is done
     hipEvent_t ev_phase[2] = {nullptr, nullptr};   // contact terms + assembly on the stream: start, end
     bool use_graphs = true;          // ADB_PCG_GRAPH=0 turns graph capture off
-    // one captured PCG batch per form of the update kernel (without and with
-    // tree groups): a step in which contacts come and go alternates between them
-    static constexpr int PCG_GRAPH_KEYS = 19, PCG_FORMS = 2;
+    // one captured PCG batch per form of the update kernel (no tree groups, with
+    // them, the others beside them): a step in which contacts come and go
+    // alternates between them
+    static constexpr int PCG_GRAPH_KEYS = 20, PCG_FORMS = 3;
     struct PcgGraph {
         hipGraphExec_t exec = nullptr;
         int batch = 0;                            // PCG batch size it was captured with
         const void* key[PCG_GRAPH_KEYS] = {};     // buffer addresses it was captured with
     } pcg_graph[PCG_FORMS];
-    double* h_scal = nullptr;        // pinned host copies of the PCG scalars (2 x 8)
+    double* h_scal = nullptr;        // pinned host copies of the PCG scalars (two)
     hipEvent_t pcg_ev[2] = {nullptr, nullptr};
     // ---- energies
     DBuf<double> epart;
@@ -267,7 +270,7 @@ struct World {
     DBuf<double> sfac;                    // per-scene factor (CCD scale, line-search alpha)
     DBuf<int> sc_goff;                    // per scene: first preconditioner group (S + 1)
     std::vector<int> h_sc_goff;
-    DBuf<double> pcg_sbb;                 // per scene: |b|^2 of the current solve
+    DBuf<double> pcg_sbb, pcg_srr;        // per scene: |b|^2 of the current solve, |r|^2 of its tree part
     double* h_sred = nullptr;             // pinned host copy of sred
     std::vector<int> h_stall_pt, h_stall_vg;
     // per-scene results of the last step

@@ -575,7 +575,7 @@ static void free_world(World& w) {
     w.h_small = nullptr;
     w.vsel.free_(); w.keepbits.free_();
     w.scene_off.free_(); w.scene_of.free_(); w.swk.free_(); w.swk_s.free_(); w.swi.free_(); w.swi_s.free_();
-    w.seg.free_(); w.sred.free_(); w.sfac.free_(); w.sc_goff.free_(); w.pcg_sbb.free_();
+    w.seg.free_(); w.sred.free_(); w.sfac.free_(); w.sc_goff.free_(); w.pcg_sbb.free_(); w.pcg_srr.free_();
     if (w.h_sred) (void)hipHostFree(w.h_sred);
     w.h_sred = nullptr;
     for (auto& r : w.prof.pending) { w.prof.pool.push_back(r.a); w.prof.pool.push_back(r.b); }
@@ -658,7 +658,7 @@ extern "C" int adb_world_create_batched(const adb_scene* s, const int* scene_off
         upload(w, w.scene_of, of.data(), w.B);
         w.sred.reserve((size_t)SRED_N * n_scenes);
         w.sfac.reserve(n_scenes);
-        w.pcg_sbb.reserve(n_scenes);
+        w.pcg_sbb.reserve(n_scenes); w.pcg_srr.reserve(n_scenes);
         w.sc_goff.reserve(n_scenes + 1);
         wait_stream(w);
     } catch (const HipError& e) {

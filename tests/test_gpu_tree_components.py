@@ -10,6 +10,7 @@ import sys
 import numpy as np
 import pytest
 
+import oracle_lib as O
 from adb_amd import scenes
 from adb_amd.capi import default_params
 from adb_amd.world import World
@@ -57,6 +58,7 @@ import sys
 import numpy as np
 sys.path[:0] = [%r, %r]
 from test_gpu_tree_components import D_HAT, column
+import oracle_lib as O
 from adb_amd import scenes
 from adb_amd.capi import default_params
 from adb_amd.world import World
@@ -88,3 +90,65 @@ def test_the_solver_graph_survives_a_changing_number_of_components(columns):
     calls = re.findall(r"\b(hip[A-Z]\w*) ?\(", r.stderr)
     assert calls.count("hipLaunchKernel") > 100
     assert 1 <= calls.count("hipGraphInstantiate") <= 2
+
+
+def wall(w, h, d=1, at=(0.0, 0.0, 0.0)):
+    s = 1.0 + GAP
+    return [(at[0] + s * i, at[1] + s * j, at[2] + s * k) for k in range(d) for j in range(h) for i in range(w)]
+
+
+LAUNCHES = """
+import sys
+sys.path[:0] = [%r, %r]
+from test_gpu_tree_components import column, one_iteration, wall
+
+st = one_iteration(column(17, 0) + wall(8, 8, at=(10.0, 0.0, 0.0)), mu=0.4)
+print("iterations", st.pcg_iters)
+"""
+
+
+def test_components_are_solved_once_beside_a_slow_one():
+    """A wall of 8 x 8 cubes, spread over several groups, takes hundreds of PCG
+    iterations; the column of 17 beside it is solved after a few, and the
+    update kernel that holds its solve (last template argument true or 1) is
+    not launched again in the others (the runtime's log of its launches)."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    tests = os.path.dirname(os.path.abspath(__file__))
+    r = subprocess.run([sys.executable, "-c", LAUNCHES % (os.path.dirname(tests), tests)], capture_output=True, text=True,
+                       env=dict(os.environ, AMD_LOG_LEVEL="3", ADB_PCG_GRAPH="0"))
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert int(re.search(r"iterations (\d+)", r.stdout).group(1)) > 50
+    updates = re.findall(r"ShaderName : .*k_pcg_update<([^>]*)>", r.stderr)
+    trees = [u for u in updates if u.split(",")[-1].strip() in ("true", "1")]
+    assert len(updates) > 50 and 1 <= len(trees) <= 8
+
+
+@pytest.mark.parametrize("batched", [False, True])
+@pytest.mark.parametrize("psd", [1, 0])
+def test_direction_beside_other_components(batched, psd):
+    """Columns of 17 and 40 (block factors), a wall of 8 x 8 and a block of 4 x 4
+    x 2 (several groups each), a column of 12, single cubes: the direction
+    against the oracle's direct solve of each component, 1e-7 of the largest
+    entry as for components alone; batched, also with scenes that hold one kind
+    only."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    parts = [column(17, 1), wall(8, 8), column(40, 2), wall(4, 4, 2), column(12, 3), [(0.0, 0.0, 0.0)]]
+    v, f, e = scenes.cube_mesh()
+    p = default_params(d_hat=D_HAT, enable_ground=0, mu=0.4, psd=psd)
+    rng = np.random.default_rng(5)
+    bodies, want = [], []
+    for k, part in enumerate(parts):
+        mine = [dict(verts=v, tris=f, edges=e, R=np.eye(3), p=(x + 16.0 * k, y, z), mass=rng.uniform(500.0, 2000.0)) for x, y, z in part]
+        ro, do = O.OracleWorld(scenes.build_scene(mine), p).newton_direction()
+        assert ro == 0
+        bodies += mine
+        want.append(do.reshape(-1, 12))
+    n = np.cumsum([0] + [len(q) for q in parts])
+    # scenes: the first column; the wall and the second column; the rest
+    w = World(scenes.build_scene(bodies), p, [0, n[1], n[3], n[6]] if batched else None)
+    rc, dq = w.newton_direction()
+    assert rc == 0
+    for a, b, d in zip(n[:-1], n[1:], want):
+        np.testing.assert_allclose(dq.reshape(-1, 12)[a:b], d, rtol=0, atol=1e-7 * np.abs(d).max())
