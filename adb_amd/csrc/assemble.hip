@@ -210,8 +210,12 @@ __global__ void k_chunk_owner(int npb, const int* __restrict__ npd, const int* _
 // host's copy of the pair lists in one workgroup (the launches of the kernels
 // above cost more than their work there).  For worlds whose body lists fit its
 // LDS; beyond, one workgroup takes several passes over them in global memory
-// (27 000 bodies 282 us, against 50 us for the kernels above).
-constexpr int STRUCT_T = 1024;
+// (27 000 bodies 282 us, against 50 us for the kernels above).  And of at most
+// STRUCT_NP body pairs: a direction of two crossed layers of rods, where every
+// pair is in contact, takes in one workgroup / by the kernels above 1.98 / 2.01
+// ms at 5600 pairs, 2.24 / 2.24 at 8500, 2.84 / 2.79 at 14 400, 4.80 / 4.44 at
+// 40 000, 8.46 / 7.56 at 90 000 and 32.8 / 28.6 at 360 000.
+constexpr int STRUCT_T = 1024, STRUCT_NP = 8192;
 // exclusive scan of in[0, n) into out[0, n], out[n] = the total, by one
 // workgroup of STRUCT_T threads (contiguous ranges per thread); returns the total
 __device__ int block_scan_excl(const int* in, int* out, int n, int* sh) {
@@ -1202,7 +1206,7 @@ void assemble_structure(World& w, bool forked) {
     const int max_chunks = (np + nc / PCH + 7) / 8 * 8;
     w.chunk_blk.reserve(std::max(max_chunks, 1));
     w.chunk_part.reserve(PART * (size_t)std::max(max_chunks, 1));
-    const bool one_wg = B + 1 <= STRUCT_LB && !w.general_paths;
+    const bool one_wg = B + 1 <= STRUCT_LB && np <= STRUCT_NP && !w.general_paths;
     if (one_wg) {
         // 3. block rows, vertex-ground starts and chunks in one workgroup
         w.pair_pack.reserve(3 * (size_t)np + 2);
