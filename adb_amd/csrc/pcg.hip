@@ -502,7 +502,9 @@ template <bool FIRST> static void launch_update(World& w, int part, int k, doubl
     };
     auto form = [&](auto f) {
         constexpr int F = decltype(f)::value;
-        if (FIRST || nbS <= 64) go(k_pcg_update<FIRST, 1, false, F>);
+        // (FIRST sums nothing)
+        if constexpr (FIRST) go(k_pcg_update<true, 1, false, F>);
+        else if (nbS <= 64) go(k_pcg_update<FIRST, 1, false, F>);
         else if (nbS <= 512) go(k_pcg_update<FIRST, 8, false, F>);
         else go(k_pcg_update<FIRST, 8, true, F>);
     };
