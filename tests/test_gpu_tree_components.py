@@ -152,3 +152,21 @@ def test_direction_beside_other_components(batched, psd):
     assert rc == 0
     for a, b, d in zip(n[:-1], n[1:], want):
         np.testing.assert_allclose(dq.reshape(-1, 12)[a:b], d, rtol=0, atol=1e-7 * np.abs(d).max())
+
+
+def bricks(w, h):
+    """Running bond: each cube rests on two of the row below."""
+    return [((1.0 + 3.0 * GAP) * i + (0.5 if j % 2 else 0.0), (1.0 + GAP) * j, 0.0) for j in range(h) for i in range(w)]
+
+
+@pytest.mark.parametrize("pos,exact", [(column(17, 0), True), (column(256, 1), True), (wall(3, 6), True), (wall(4, 10), True), (bricks(6, 6), True),
+                                       (column(16, 2), False), (column(257, 3), False), (wall(4, 4, 4), False)],
+                         ids=["path17", "path256", "wall3x6", "wall4x10", "bricks6x6", "path16", "path257", "block4x4x4"])
+def test_factored_components_are_solved_at_once(pos, exact):
+    """A component with factors is solved exactly: 1 iteration in exact
+    arithmetic, 3 allowed for the rounding of the stiff contacts (a NumPy model:
+    at most 3 at distances down to 1e-9).  One that is spread over several
+    groups of 8 is not solved in so few."""
+    st = one_iteration(pos, mu=0.4)
+    assert st.n_pt + st.n_ee > 0 and st.pcg_not_converged == 0
+    assert 1 <= st.pcg_iters <= 3 if exact else st.pcg_iters > 6
