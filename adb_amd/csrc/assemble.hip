@@ -858,9 +858,7 @@ __global__ __launch_bounds__(256) void k_group_inv(const int* __restrict__ list,
 // with npd the count on the device); build_groups reads the count with them.
 static void groups_fetch(World& w, int npb, const int* npd, const int* pack, hipStream_t st) {
     if (3 * (size_t)npb + 2 > w.h_pairs_cap) {
-        if (w.h_pairs) ADB_HIP(hipHostFree(w.h_pairs));
-        w.h_pairs_cap = 3 * (size_t)npb + 2 + (size_t)npb / 2 + 64;
-        ADB_HIP(hipHostMalloc((void**)&w.h_pairs, w.h_pairs_cap * sizeof(int), hipHostMallocDefault));
+        regrow_pinned(w.h_pairs, w.h_pairs_cap, 3 * (size_t)npb + 2 + (size_t)npb / 2 + 64);
     }
     if (!w.ev_pairs) ADB_HIP(hipEventCreateWithFlags(&w.ev_pairs, hipEventDisableTiming));
     w.h_pairs_n = npb;
@@ -1054,9 +1052,7 @@ static void build_groups(World& w) {
     if (!w.ev_grp) ADB_HIP(hipEventCreateWithFlags(&w.ev_grp, hipEventDisableTiming));
     wait_event(w, w.ev_grp);
     if (total > w.h_grp_pack_cap) {
-        if (w.h_grp_pack) ADB_HIP(hipHostFree(w.h_grp_pack));
-        w.h_grp_pack_cap = total + total / 2 + 64;
-        ADB_HIP(hipHostMalloc((void**)&w.h_grp_pack, w.h_grp_pack_cap * sizeof(long long), hipHostMallocDefault));
+        regrow_pinned(w.h_grp_pack, w.h_grp_pack_cap, total + total / 2 + 64);
         std::memset(w.h_grp_pack, 0, w.h_grp_pack_cap * sizeof(long long));
     }
     w.grp_pack.reserve(total);
@@ -1086,12 +1082,7 @@ static void build_groups(World& w) {
     if (w.n_trees > 0) {
         // the tree groups' tables, in a buffer that moves only when it grows
         const size_t nt = w.hg_tabs.size();
-        if (nt > w.h_tree_pin_cap) {
-            if (w.h_tree_pin) ADB_HIP(hipHostFree(w.h_tree_pin));
-            w.h_tree_pin = nullptr;
-            w.h_tree_pin_cap = nt + nt / 2;
-            ADB_HIP(hipHostMalloc((void**)&w.h_tree_pin, w.h_tree_pin_cap * sizeof(int), hipHostMallocDefault));
-        }
+        if (nt > w.h_tree_pin_cap) regrow_pinned(w.h_tree_pin, w.h_tree_pin_cap, nt + nt / 2);
         std::memcpy(w.h_tree_pin, w.hg_tabs.data(), nt * sizeof(int));
         w.tree_pack.reserve(nt);
         ADB_HIP(hipMemcpyAsync(w.tree_pack.p, w.h_tree_pin, nt * sizeof(int), hipMemcpyHostToDevice, w.stream));

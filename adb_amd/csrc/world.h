@@ -35,13 +35,27 @@ template <class T> struct DBuf {
     T* p = nullptr; size_t cap = 0;
     void reserve(size_t n) {
         if (n <= cap) return;
-        if (p) ADB_HIP(hipFree(p));
+        void* old = p;
+        p = nullptr; cap = 0;            // empty if the allocation fails
+        if (old) ADB_HIP(hipFree(old));
         size_t c = n + n / 2 + 64;
-        ADB_HIP(hipMalloc((void**)&p, c * sizeof(T)));
-        cap = c;
+        T* q = nullptr;
+        ADB_HIP(hipMalloc((void**)&q, c * sizeof(T)));
+        p = q; cap = c;
     }
     void free_() { if (p) (void)hipFree(p); p = nullptr; cap = 0; }
 };
+
+// Pinned host buffer p of c entries in place of the old one; empty if the
+// allocation fails.
+template <class T> void regrow_pinned(T*& p, size_t& cap, size_t c) {
+    void* old = p;
+    p = nullptr; cap = 0;
+    if (old) ADB_HIP(hipHostFree(old));
+    T* q = nullptr;
+    ADB_HIP(hipHostMalloc((void**)&q, c * sizeof(T), hipHostMallocDefault));
+    p = q; cap = c;
+}
 
 // Compact body-space record of one PT/EE contact (doubles).  With D the
 // dimension of the contact's translation-free point space (3, 6 or 9; 0 when

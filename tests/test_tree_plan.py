@@ -31,6 +31,13 @@ extern "C" int plan(int n, int m, const int* pairs, const int* bodies, int* out,
     return (int)t.size() - 3;
 }
 extern "C" int solve_ints(int n, int nlev, int ne) { return tree_solve_ints(n, nlev, ne); }
+// capacity left behind by a pinned buffer whose growth fails; -1: it did not fail
+extern "C" int pinned_after_failure(int cap0) {
+    int* p = nullptr;
+    size_t cap = cap0;
+    try { regrow_pinned(p, cap, (size_t)1 << 50); } catch (const HipError&) { return p ? -2 : (int)cap; }
+    return -1;
+}
 """
 
 
@@ -177,3 +184,7 @@ def test_components_that_fill_in_are_refused(lib, name):
 def test_a_path_takes_logarithmic_rounds(lib):
     n, pairs = path(256)
     assert fields(lib, plan(lib, n, pairs, np.arange(n)))["nlev"] <= 2 * 8 + 1
+
+
+def test_a_failed_pinned_growth_leaves_no_capacity(lib):
+    assert lib.pinned_after_failure(100) == 0
