@@ -750,9 +750,6 @@ __device__ __forceinline__ void contact_small(const WorldArgs& a, const Stage& s
 // (a scheduling barrier after each rotation keeps the live ranges to one
 // rotation).  Split this way the geometry's registers stay out of the Jacobi
 // kernel, and the matrix of a contact is built by nine threads at once.
-__host__ __device__ constexpr int P9(int p, int q) {
-    return p <= q ? p * 9 - p * (p - 1) / 2 + (q - p) : q * 9 - q * (q - 1) / 2 + (p - q);
-}
 constexpr int C3_ROLES = 10;
 struct C3Ctx {
     Geo G;
@@ -884,71 +881,20 @@ __device__ __forceinline__ void c3_fields(const WorldArgs& a, int cid, const C3C
 }
 __device__ __forceinline__ void psd9(const WorldArgs& a, int cid) {
     double* R = a.rec + REC * (size_t)cid;
-    // PK: packed K and V in registers (static indices); a scheduling barrier
-    // after each rotation keeps the live ranges to one rotation
-    double A[45];
+    double A[45], V[81];
 #pragma unroll
     for (int p = 0; p < 9; p++)
 #pragma unroll
-        for (int q = p; q < 9; q++) A[P9(p, q)] = R[R_PK + 9 * p + q];
-    {
-        double Vr[81];
+        for (int q = p; q < 9; q++) A[PK_<9>(p, q)] = R[R_PK + 9 * p + q];
+    jacobi_packed<9>(A, V);
+    project_packed<9>(A, V);
 #pragma unroll
-        for (int e = 0; e < 81; e++) Vr[e] = (e % 10 == 0) ? 1.0 : 0.0;
-        for (int sweep = 0; sweep < MAX_SWEEPS; sweep++) {
-            double off = 0.0, tot = 0.0;
+    for (int p = 0; p < 9; p++)
 #pragma unroll
-            for (int p = 0; p < 9; p++)
-#pragma unroll
-                for (int q = p; q < 9; q++) {
-                    const double x = A[P9(p, q)] * A[P9(p, q)];
-                    if (p == q) tot += x; else { off += 2.0 * x; tot += 2.0 * x; }
-                }
-            if (off <= JACOBI_TOL * tot || off == 0.0) break;
-            const double thr = JACOBI_SKIP * sqrt(tot);
-#pragma unroll
-            for (int p = 0; p < 8; p++)
-#pragma unroll
-                for (int q = p + 1; q < 9; q++) {
-                    const double apq = A[P9(p, q)];
-                    if (fabs(apq) > thr) {
-                        const double app = A[P9(p, p)], aqq = A[P9(q, q)];
-                        double c, s, t;
-                        jacobi_cs(app, aqq, apq, c, s, t);
-#pragma unroll
-                        for (int k = 0; k < 9; k++) {
-                            if (k == p || k == q) continue;
-                            const double akp = A[P9(k, p)], akq = A[P9(k, q)];
-                            A[P9(k, p)] = fma(c, akp, -s * akq);
-                            A[P9(k, q)] = fma(s, akp, c * akq);
-                        }
-                        A[P9(p, p)] = fma(-t, apq, app);
-                        A[P9(q, q)] = fma(t, apq, aqq);
-                        A[P9(p, q)] = 0.0;
-#pragma unroll
-                        for (int k = 0; k < 9; k++) {
-                            const double vkp = Vr[9 * k + p], vkq = Vr[9 * k + q];
-                            Vr[9 * k + p] = fma(c, vkp, -s * vkq);
-                            Vr[9 * k + q] = fma(s, vkp, c * vkq);
-                        }
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+        for (int q = p; q < 9; q++) {
+            R[R_PK + 9 * p + q] = A[PK_<9>(p, q)];
+            R[R_PK + 9 * q + p] = A[PK_<9>(p, q)];
         }
-        double wv[9];
-#pragma unroll
-        for (int k = 0; k < 9; k++) wv[k] = fmax(A[P9(k, k)], 0.0);
-#pragma unroll
-        for (int p = 0; p < 9; p++)
-#pragma unroll
-            for (int q = p; q < 9; q++) {
-                double s = 0.0;
-#pragma unroll
-                for (int k = 0; k < 9; k++) s += Vr[9 * p + k] * wv[k] * Vr[9 * q + k];
-                R[R_PK + 9 * p + q] = s;
-                R[R_PK + 9 * q + p] = s;
-            }
-    }
 }
 // The roles and the Jacobi are separate kernels, so the role threads get the
 // registers of their own code (two wavefronts per SIMD) while the Jacobi
