@@ -28,11 +28,10 @@
 // through differences, so the Hessian annihilates rigid translations.  With
 // Q = h (x) I3, h the Helmert basis of the complement of (1, ..., 1) over the
 // contact's points, H = Q^T (Q H Q^T) Q and the projection onto the PSD cone
-// is Q^T P(Q H Q^T) Q: a D x D symmetric eigenproblem.  The kernel API, as in
-// the reference, returns a Hessian whose eigenvalues are all >= 0 unchanged;
-// the world path always rebuilds V diag(max(w, 0)) V^T, equal to it within
-// the Jacobi tolerance (the reference's own test sees the nine rounding-level
-// eigenvalues of the translations).
+// is Q^T P(Q H Q^T) Q: a D x D symmetric eigenproblem.  Both paths always
+// rebuild V diag(max(w, 0)) V^T; where the reference returns a Hessian whose
+// eigenvalues are all >= 0 unchanged (its test sees the rounding-level
+// eigenvalues of the translations) that equals it within the Jacobi tolerance.
 //
 // Kernel-level API (the abdtk functions): k_hess_api, one thread per contact
 // in the five-coordinate frame of terms.h; mollified edge pairs in
@@ -1287,9 +1286,9 @@ void contact_terms(World& w) {
                 ADB_HIP(hipGetLastError());
             }
             ADB_HIP(hipEventRecord(w.ev_side[1], w.stream2));
-            // the 6x6 projections of the 3-point contacts (VALU-bound) on a third
-            // stream, beside the 2- and 3-point record kernels (bound by their
-            // scattered loads and stores); they write disjoint record fields
+            // the 3x3 projections of the 3-point contacts and the 4-point records on
+            // a third stream, beside the 2- and 3-point record kernels (bound by
+            // their scattered loads and stores); they write disjoint record fields
             ADB_HIP(hipStreamWaitEvent(w.stream3, w.ev_side[0], 0));
             {
                 // per 3-point contact: ids, 4 points, type and distance in; PK (36 doubles)

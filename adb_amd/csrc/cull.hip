@@ -403,11 +403,12 @@ __global__ __launch_bounds__(256) void k_sweep_pairs(int B, const unsigned long 
 //      segment, from which the line search's trial sets are filtered.
 // Boxes only cull; the FP64 predicate decides, so the sets equal those of the
 // all-pairs tests (model/thread_local_culling.cpp:209-386 pt/ee_col_set_task).
-// Fewest edges of a slice of the EE pass, one round of the workgroup's
-// threads: each slice stages the other body's edges again, which for small
+// Edges per slice of the EE pass from which on a mesh is split once more, into
+// ceil(edges / EE_SLICE) equal slices (so of more than EE_SLICE / 2 edges each) up
+// to ee_slices: each slice stages the other body's edges again, which for small
 // meshes costs more than the tests it splits (cards of 18 edges, 9900 pairs: 515
 // us in 4 slices, 410 us in one; cubes and spheres of 480 edges in 256 scenes, swept
-// boxes: 650 us in 4, 586 us in two)
+// boxes: 650 us in 4, 586 us in two of 240)
 constexpr int EE_SLICE = NB_THREADS;
 constexpr int PAIRS_PT = 4;                    // box tests per thread per round
 // workgroups per body pair: 2 PT passes + the EE pass in ee_slices slices (tuning)

@@ -157,10 +157,9 @@ __device__ __forceinline__ d3 pick(d3 p0, d3 p1, d3 p2, d3 p3, int k) {
 __device__ __forceinline__ d3 unit(d3 a) { double l = sqrt(sqn(a)); return mk(a.x / l, a.y / l, a.z / l); }
 
 // The frame of a contact: separation sum_k gam_k x_k = delta n, tangents f1,
-// f2, and the weights of the two normal functionals m1, m2 (see above).  The
-// tangents are also the contact's friction basis (model/pt_ipc.cpp:31-103,
-// model/ee_ipc.cpp:38-110): the edge (PL), the first edge (PLANE), or
-// basis_pp's choice (PP), and n x f1 or f1 x n.
+// f2, and the weights of the two normal functionals m1, m2 (see above).  f1 is
+// the edge (PL), the first edge (PLANE) or any tangent (PP).  (Friction has its
+// own basis, of the reference's signs: friction_frame.)
 struct Frame {
     int kind;
     unsigned in;                 // bit k: point k takes part
@@ -227,7 +226,7 @@ __device__ __forceinline__ void contact_frame(int is_ee, int type, d3 P0, d3 P1,
         if (kind == K_PL) {
             F.f2 = cross(F.f1, F.n);
         } else {
-            // basis_pp of the reference: the larger of x x n and y x n
+            // the larger of x x n and y x n
             const d3 cx = mk(0.0, -F.n.z, F.n.y), cy = mk(F.n.z, 0.0, -F.n.x);
             F.f1 = unit(sqn(cx) > sqn(cy) ? cx : cy);
             F.f2 = cross(F.n, F.f1);

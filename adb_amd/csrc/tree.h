@@ -27,13 +27,18 @@
 
 namespace adb {
 
-// Components of at most TREE_MIN bodies keep two or three small groups: a few
-// iterations, and the iteration counts that callers see there stay.
+// Components of at most TREE_MIN bodies keep two or three small groups, so that
+// the iteration counts which callers (and the tests of truncated solves) see
+// on small stacks stay what they were.  Speed is no reason: with factors from 9
+// bodies on a direction of one column of 10 cubes takes 326 us instead of 483,
+// of 200 of them 636 instead of 2258, of 80 walls of 3 x 4 717 instead of 1198.
 constexpr int TREE_MIN = 16;
 constexpr int TREE_MAX = 256;        // bodies of a component: its vector stays in LDS
 constexpr int TREE_DEG = 8;          // neighbours of a body when it is eliminated
 constexpr int TREE_FILL = 6;         // blocks below the diagonal per body
-constexpr int TREE_MIN_ITER = 16;    // iteration limits below this keep the small groups
+// iteration limits below this keep the small groups, whose truncated iterates
+// (and reports of them) are what a caller with such a limit has asked for
+constexpr int TREE_MIN_ITER = 16;
 
 // One component's table, ints from T on.  A "block" e is a block below the
 // diagonal of column own[e], row node[e] (positions), blocks in column order.

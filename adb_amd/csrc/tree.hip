@@ -3,8 +3,8 @@
 // round: the bodies of a round are independent, and what bounds it is the
 // chain D_j -> L_j -> V_ij (three barriers, the 12 pivots of L_j the longest
 // link), not the few hundred blocks of 1.2 KB a component reads and writes.
-// Two chains of 32 tori (5 rounds) 90 us and 100 rows of 100 cards (7 rounds)
-// 206 us, against 73 and 264 us for the explicit inverses of groups of 8 that
+// Two chains of 32 tori (5 rounds) 80 us and 100 rows of 100 cards (7 rounds)
+// 180 us, against 73 and 264 us for the explicit inverses of groups of 8 that
 // left 160 and 124 PCG iterations (9 and 32 us each).
 //
 // A pivot that is not positive and finite (a matrix that is not positive

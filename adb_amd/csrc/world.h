@@ -183,7 +183,7 @@ struct World {
     DBuf<int> ccls;                  // class per contact: 0 inactive, 1..3 = D / 3
     DBuf<double> cdist;              // squared distance per contact
     DBuf<int> clist;                 // class 1 from the front, class 2 from the back
-    DBuf<int> clist3;                // class 3 contacts
+    DBuf<int> clist3;                // class 3 from the front, class 4 from the back
     DBuf<int> ccount;                // class 1..4 sizes, chunk count
     DBuf<double> ctk;                // TKN per PT/EE contact: lagged friction basis (see TKN)
     DBuf<double> clam;               // 1 per PT/EE contact
