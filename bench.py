@@ -157,6 +157,14 @@ FP64_OPS_JSON = os.path.join(ROOT, "profiles", "fp64_ops_2000_icospheres.json")
 FP64_OPS_OF_SCOPE = {"contact_group", "contact_pk", "narrow_set", "narrow_ccd"}
 
 
+def dominant_scope(ranked):
+    """The scope that the roofline is quoted for, of (name, profile) pairs by
+    decreasing device time: the first on the main stream.  A side stream's
+    scope is no part of the step's critical path, and its event time includes
+    the kernels that it shares the GPU with."""
+    return next(((k, v) for k, v in ranked if v["launches"] > 0 and k not in SIDE_SCOPES), None)
+
+
 def measured_fp64_ops(scope, launches):
     """FP64 operations of `launches` launches of the scope from the committed
     counter summary, when it was measured on this workload and launch count."""
@@ -394,14 +402,13 @@ def main():
                  "newton_iters": t2["newton"], "pcg_iters": t2["pcg"]}
 
     steps_per_s = args.steps / elapsed
-    # dominant kernel scope: the most device time in the profiled steps (side
-    # stream scopes included; their event times include sharing the GPU with
-    # the main stream's kernels).  FP64-VALU-bound scopes with a counted
+    # dominant kernel scope: the most device time on the main stream in the
+    # profiled steps.  FP64-VALU-bound scopes with a counted
     # operation total report FP64 throughput against 78.6 TFLOP/s (MI355X's
     # FP64 peak, the same for vector and matrix); the others report their
     # algorithmic HBM bytes against 8 TB/s.
     ranked = sorted(prof.items(), key=lambda kv: -kv[1]["ms"])
-    dom = next(((k, v) for k, v in ranked if v["launches"] > 0), None)
+    dom = dominant_scope(ranked)
     roofline = None
     if dom:
         k, v = dom
@@ -417,14 +424,14 @@ def main():
                         "peak": MI355X_FP64_TFLOPS, "unit": "TFLOP/s", "frac": round(tf / MI355X_FP64_TFLOPS, 4),
                         "traffic": None, "avg_launch_ms": avg_ms, "flops_per_launch": per, "launches": v["launches"],
                         "flops_source": "counted" if v.get("flops", 0.0) > 0.0 else "rocprofv3 FP64 instruction counters",
-                        "on_side_stream": k in SIDE_SCOPES, "concurrent_side_stream_ms": side}
+                        "on_side_stream": False, "concurrent_side_stream_ms": side}
         else:
             bytes_per_launch = v["bytes"] / v["launches"]
             gbs = bytes_per_launch / (avg_ms * 1e-3) / 1e9
             roofline = {"kernel": k, "bound": "hbm", "achieved": round(gbs, 1), "peak": MI355X_HBM_GBS,
                         "unit": "GB/s", "frac": round(gbs / MI355X_HBM_GBS, 4), "traffic": None,
                         "avg_launch_ms": avg_ms, "bytes_per_launch": bytes_per_launch, "launches": v["launches"],
-                        "on_side_stream": k in SIDE_SCOPES, "concurrent_side_stream_ms": side}
+                        "on_side_stream": False, "concurrent_side_stream_ms": side}
         # HBM bytes per launch measured by rocprofv3 --pmc on this workload (committed summary)
         if os.path.exists(TRAFFIC_JSON):
             with open(TRAFFIC_JSON) as fh:
