@@ -199,7 +199,7 @@ __global__ void k_pair_chunks(int npb, const int* __restrict__ npd, const int* _
 // chunk_off = exclusive scan of nch (npb + 1 entries); the chunk count also
 // goes to counts[4] for the byte accounting.  Each chunk looks its pair up: a
 // thread that writes all of a pair's chunks takes as long as the largest pair
-// has (2500 crowded bodies, 4.6e4 chunks: 10.5 -> 5.5 us; 90 000 pairs of one
+// has (2500 crowded bodies, 2.7e4 chunks: 10.5 -> 5.5 us; 90 000 pairs of one
 // chunk 5.2 -> 7.0)
 __global__ void k_chunk_owner(int npb, const int* __restrict__ npd, const int* __restrict__ chunk_off, int* __restrict__ chunk_pair,
                               int* __restrict__ counts) {
