@@ -660,8 +660,10 @@ static int solve_part(World& w, int part, double* dq_out, int* iters, const std:
 // the rest, where some component is spread over several groups, takes tens
 // or hundreds, each of which would repeat the tree solves (8 x 8 cubes in a
 // wall, 214 iterations, beside a column of 17: 5137 us a direction against 2790
-// in two parts, 3132 with groups of 8 throughout).  The residual test is that
+// in two parts, 3100 with groups of 8 throughout).  The residual test is that
 // of the whole: the second part adds what the first left to both its sides.
+// Each part has the iteration limit to itself, so that none is refused for the
+// other's iterations; the count returned is their sum.
 int pcg_solve(World& w, double* dq_out, int* iters, const std::function<void()>& after, bool* after_valid) {
     if (after_valid) *after_valid = false;
     int it = 0, rc;
